@@ -25,7 +25,7 @@ WALK_SOURCE = CSRC / "kvr_module_walk.c"
 WALK_OUTPUT = PACKAGE_ROOT / "kv_cache_repair_amd" / ("_kvr_walk" + sysconfig.get_config_var("EXT_SUFFIX"))
 LAYOUT_SOURCE = CSRC / "kvr_tensor_layout.cpp"
 LAYOUT_OUTPUT = PACKAGE_ROOT / "kv_cache_repair_amd" / ("_kvr_layout" + sysconfig.get_config_var("EXT_SUFFIX"))
-SOURCES = ("kvr_common.hip", "kvr_rotate.hip", "kvr_scatter.hip", "kvr_fresh.hip", "kvr_layer.hip", "kvr_gemm.hip", "kvr_attention.hip", "kvr_decoder.hip", "kvr_writeback.hip", "kvr_inputs.hip", "kvr_scoring.hip")
+SOURCES = ("kvr_common.hip", "kvr_rotate.hip", "kvr_scatter.hip", "kvr_fresh.hip", "kvr_layer.hip", "kvr_gemm.hip", "kvr_gemm_tiled.hip", "kvr_attention.hip", "kvr_decoder.hip", "kvr_writeback.hip", "kvr_inputs.hip", "kvr_scoring.hip")
 ARCH = "gfx950"
 
 # Packed-FP32 instructions are disabled: hipcc still vectorises ordinary

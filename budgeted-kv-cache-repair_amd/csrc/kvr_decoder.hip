@@ -20,6 +20,12 @@
 // reduce launches, whose sums are read straight from the partials by the next
 // kernel (RoPE + scatter, residual + post-attention norm, residual + the next
 // layer's input norm), with the reduce kernel's summation order and rounding.
+//
+// kvr_decoder_tiled_* is the same layer over the tiled projection kernel
+// (kvr_gemm_tiled.hip) for more than 64 rows, where the module path took ~20
+// Python-dispatched launches per layer (seven library GEMMs, SiLU product,
+// residual adds): at 71 rows of a 32-layer 8B model the host could not issue
+// them as fast as the GPU ran them.
 #include "kvr_internal.h"
 
 namespace kvr {
@@ -58,42 +64,54 @@ ScratchLayout scratch_layout(const kvr_refresh_desc* d) {
     return s;
 }
 
-int check_refresh(const kvr_refresh_desc* d) {
+// Which projection kernel a forward runs: the streaming kernel (at most 64
+// rows, kvr_decoder_*) or the tiled one (kvr_decoder_tiled_*).
+struct Projections {
+    bool tiled;
+
+    int64_t workspace(int32_t m, int32_t rows, int32_t k) const {
+        return tiled ? tiled_workspace_bytes(m, rows, k) : kvr_linear_workspace_bytes(m, rows, k);
+    }
+    int run(const void* x, int32_t n_weights, const void* const* w, const int32_t* rows, const int64_t* ldw, void* y,
+            int32_t m, int32_t k, int64_t ldx, int64_t ldy, int32_t epilogue, const void* residual, int64_t ldr,
+            void* ws, int64_t ws_bytes, int32_t dtype, void* stream, bool reduce, int32_t* splits) const {
+        return (tiled ? tiled_linear : linear_multi)(x, n_weights, w, rows, ldw, y, m, k, ldx, ldy, epilogue, residual,
+                                                     ldr, ws, ws_bytes, dtype, stream, reduce, splits);
+    }
+};
+
+int check_refresh(const kvr_refresh_desc* d, bool tiled) {
     if (!d) return KVR_E_NULL_POINTER;
     if (d->dtype != KVR_DTYPE_BF16 && d->dtype != KVR_DTYPE_F16) return KVR_E_UNSUPPORTED_DTYPE;
-    if (d->rows <= 0 || d->rows > 64 || d->hidden <= 0 || d->q_heads <= 0 || d->kv_heads <= 0 ||
+    if (d->rows <= 0 || d->rows > (tiled ? kTiledMaxRows : 64) || d->hidden <= 0 || d->q_heads <= 0 || d->kv_heads <= 0 ||
         d->q_heads % d->kv_heads || d->head_dim <= 0 || d->head_dim % 2 || d->intermediate <= 0 || d->n_keys <= 0)
         return KVR_E_UNSUPPORTED_SHAPE;
     const int64_t qd = static_cast<int64_t>(d->q_heads) * d->head_dim;
     // every projection's k (hidden, q_heads * head_dim, intermediate) must be a multiple of 8
     if (d->hidden % 8 || qd % 8 || d->intermediate % 8 || (d->kv_heads * d->head_dim) % 8)
         return KVR_E_UNSUPPORTED_SHAPE;
+    if (tiled && (d->hidden % 64 || qd % 64 || d->intermediate % 64)) return KVR_E_UNSUPPORTED_SHAPE;
     if (!(d->scale > 0.f) && !(d->scale < 0.f)) return KVR_E_INVALID_ARGUMENT;
     return KVR_OK;
 }
 
 int64_t max_of(int64_t a, int64_t b) { return a > b ? a : b; }
 
-}  // namespace
-}  // namespace kvr
-
-using namespace kvr;
-
-extern "C" int64_t kvr_decoder_scratch_bytes(const kvr_refresh_desc* d) {
-    const int st = check_refresh(d);
+int64_t scratch_bytes(const kvr_refresh_desc* d, bool tiled) {
+    const int st = check_refresh(d, tiled);
     if (st < 0) return st;
     return scratch_layout(d).total;
 }
 
-extern "C" int64_t kvr_decoder_gemm_workspace_bytes(const kvr_refresh_desc* d) {
-    const int st = check_refresh(d);
+int64_t gemm_workspace_bytes(const kvr_refresh_desc* d, bool tiled) {
+    const int st = check_refresh(d, tiled);
     if (st < 0) return st;
+    const Projections p{tiled};
     const int32_t m = d->rows, h = d->hidden, in = d->intermediate;
     const int32_t qd = d->q_heads * d->head_dim, kd = d->kv_heads * d->head_dim;
-    const int64_t sizes[] = {
-        kvr_linear_workspace_bytes(m, qd + 2 * kd, h), kvr_linear_workspace_bytes(m, qd, h),
-        kvr_linear_workspace_bytes(m, kd, h),          kvr_linear_workspace_bytes(m, h, qd),
-        kvr_linear_workspace_bytes(m, 2 * in, h),      kvr_linear_workspace_bytes(m, h, in)};
+    // the tiled gate/up never splits K
+    const int64_t sizes[] = {p.workspace(m, qd + 2 * kd, h), p.workspace(m, qd, h), p.workspace(m, kd, h),
+                             p.workspace(m, h, qd), tiled ? 0 : p.workspace(m, 2 * in, h), p.workspace(m, h, in)};
     int64_t need = 0;
     for (int64_t v : sizes) {
         if (v < 0) return v;
@@ -102,8 +120,9 @@ extern "C" int64_t kvr_decoder_gemm_workspace_bytes(const kvr_refresh_desc* d) {
     return need;
 }
 
-extern "C" int kvr_decoder_layer(const kvr_layer_desc* L, const kvr_refresh_desc* d, void* hidden, void* stream) {
-    int st = check_refresh(d);
+int decoder_layer(const kvr_layer_desc* L, const kvr_refresh_desc* d, void* hidden, void* stream, bool tiled,
+                  int64_t gemm_need) {
+    int st = check_refresh(d, tiled);
     if (st < 0) return st;
     if (!L || !hidden || !d->scratch || !d->positions || !d->cos || !d->sin || !d->schedule || !d->host_schedule)
         return KVR_E_NULL_POINTER;
@@ -115,10 +134,10 @@ extern "C" int kvr_decoder_layer(const kvr_layer_desc* L, const kvr_refresh_desc
     const ScratchLayout s = scratch_layout(d);
     if (d->scratch_bytes < s.total || (reinterpret_cast<uintptr_t>(d->scratch) & (kScratchAlign - 1)))
         return KVR_E_WORKSPACE_TOO_SMALL;
-    const int64_t gemm_need = kvr_decoder_gemm_workspace_bytes(d);
     if (gemm_need < 0) return static_cast<int>(gemm_need);
     if (gemm_need > 0 && (!d->gemm_workspace || d->gemm_workspace_bytes < gemm_need))
         return KVR_E_WORKSPACE_TOO_SMALL;
+    const Projections proj{tiled};
 
     char* base = static_cast<char*>(d->scratch);
     char* normed = base + s.normed;
@@ -144,7 +163,7 @@ extern "C" int kvr_decoder_layer(const kvr_layer_desc* L, const kvr_refresh_desc
     const int64_t rows_h[4] = {h, h, h, h};
     if (!L->input_normed)
         KVR_TRY(kvr_rms_norm(hidden, nullptr, nullptr, normed, L->input_norm, m, h, rows_h, L->eps_input, dt, stream));
-    const PartialSums gemm_partials{static_cast<const float*>(gws), 0};
+    const PartialSums gemm_partials{static_cast<const float*>(gws), 0, tiled ? m : kPartialTileRows};
     const bool norm_partials = rms_norm_partials_ok(h, dt);
 
     // q/k/v projections (+ Qwen3's per-head norms: inside the fresh-row
@@ -160,7 +179,7 @@ extern "C" int kvr_decoder_layer(const kvr_layer_desc* L, const kvr_refresh_desc
         const void* w[3] = {L->w_q, L->w_k, L->w_v};
         const int32_t rows[3] = {qd, kd, kd};
         const int64_t ldw[3] = {L->ld_q, L->ld_k, L->ld_v};
-        KVR_TRY(linear_multi(normed, 3, w, rows, ldw, qkv, m, h, h, qd + 2 * kd, KVR_LINEAR_CONCAT, nullptr, 0, gws,
+        KVR_TRY(proj.run(normed, 3, w, rows, ldw, qkv, m, h, h, qd + 2 * kd, KVR_LINEAR_CONCAT, nullptr, 0, gws,
                              gwb, dt, stream, /*reduce=*/false, &qkv_splits));
         qp = qkv;
         kp = qkv + static_cast<int64_t>(qd) * 2;
@@ -170,9 +189,13 @@ extern "C" int kvr_decoder_layer(const kvr_layer_desc* L, const kvr_refresh_desc
         char* qb = qkv;
         char* kb = qkv + static_cast<int64_t>(m) * qd * 2;
         char* vb = kb + static_cast<int64_t>(m) * kd * 2;
-        KVR_TRY(kvr_linear(normed, L->w_q, qb, m, qd, h, h, L->ld_q, qd, gws, gwb, dt, stream));
-        KVR_TRY(kvr_linear(normed, L->w_k, kb, m, kd, h, h, L->ld_k, kd, gws, gwb, dt, stream));
-        KVR_TRY(kvr_linear(normed, L->w_v, vb, m, kd, h, h, L->ld_v, kd, gws, gwb, dt, stream));
+        auto one = [&](const void* w, void* y, int32_t n, int64_t ld) {
+            return proj.run(normed, 1, &w, &n, &ld, y, m, h, h, n, KVR_LINEAR_CONCAT, nullptr, 0, gws, gwb, dt, stream,
+                            /*reduce=*/true, nullptr);
+        };
+        KVR_TRY(one(L->w_q, qb, qd, L->ld_q));
+        KVR_TRY(one(L->w_k, kb, kd, L->ld_k));
+        KVR_TRY(one(L->w_v, vb, kd, L->ld_v));
         const int64_t rows_d[4] = {dim, dim, dim, dim};
         char* qn = base + s.qn;
         char* kn = base + s.kn;
@@ -222,7 +245,7 @@ extern "C" int kvr_decoder_layer(const kvr_layer_desc* L, const kvr_refresh_desc
         const int32_t rows[1] = {h};
         const int64_t ldw[1] = {L->ld_o};
         int32_t splits = 1;
-        KVR_TRY(linear_multi(attn, 1, w, rows, ldw, o_out, m, qd, qd, h, KVR_LINEAR_CONCAT, nullptr, 0, gws, gwb, dt,
+        KVR_TRY(proj.run(attn, 1, w, rows, ldw, o_out, m, qd, qd, h, KVR_LINEAR_CONCAT, nullptr, 0, gws, gwb, dt,
                              stream, /*reduce=*/!norm_partials, &splits));
         if (norm_partials && splits > 1) {
             PartialSums p = gemm_partials;
@@ -239,18 +262,18 @@ extern "C" int kvr_decoder_layer(const kvr_layer_desc* L, const kvr_refresh_desc
     const void* gw[2] = {L->w_gate, L->w_up};
     const int32_t gr[2] = {in, in};
     const int64_t gl[2] = {L->ld_gate, L->ld_up};
-    KVR_TRY(kvr_linear_multi(normed, 2, gw, gr, gl, act, m, h, h, in, KVR_LINEAR_SILU_GATE, nullptr, 0, gws, gwb, dt,
-                             stream));
+    KVR_TRY(proj.run(normed, 2, gw, gr, gl, act, m, h, h, in, KVR_LINEAR_SILU_GATE, nullptr, 0, gws, gwb, dt, stream,
+                     /*reduce=*/true, nullptr));
     const void* dw[1] = {L->w_down};
     const int32_t dr[1] = {h};
     const int64_t dl[1] = {L->ld_down};
     if (!L->next_norm) {
-        KVR_TRY(kvr_linear_multi(act, 1, dw, dr, dl, hidden, m, in, in, h, KVR_LINEAR_RESIDUAL, hidden2, h, gws, gwb,
-                                 dt, stream));
+        KVR_TRY(proj.run(act, 1, dw, dr, dl, hidden, m, in, in, h, KVR_LINEAR_RESIDUAL, hidden2, h, gws, gwb, dt,
+                         stream, /*reduce=*/true, nullptr));
     } else {  // ... and the next layer's input norm into `normed`
         int32_t splits = 1;
         if (norm_partials) {
-            KVR_TRY(linear_multi(act, 1, dw, dr, dl, o_out, m, in, in, h, KVR_LINEAR_CONCAT, nullptr, 0, gws, gwb, dt,
+            KVR_TRY(proj.run(act, 1, dw, dr, dl, o_out, m, in, in, h, KVR_LINEAR_CONCAT, nullptr, 0, gws, gwb, dt,
                                  stream, /*reduce=*/false, &splits));
         }
         if (norm_partials && splits > 1) {
@@ -260,8 +283,8 @@ extern "C" int kvr_decoder_layer(const kvr_layer_desc* L, const kvr_refresh_desc
                                       stream));
         } else {
             if (!norm_partials)
-                KVR_TRY(kvr_linear_multi(act, 1, dw, dr, dl, hidden, m, in, in, h, KVR_LINEAR_RESIDUAL, hidden2, h,
-                                         gws, gwb, dt, stream));
+                KVR_TRY(proj.run(act, 1, dw, dr, dl, hidden, m, in, in, h, KVR_LINEAR_RESIDUAL, hidden2, h, gws, gwb,
+                                 dt, stream, /*reduce=*/true, nullptr));
             else  // one split: the projection was written to o_out
                 KVR_TRY(kvr_rms_norm(o_out, hidden2, hidden, normed, L->next_norm, m, h, rows_h, L->eps_next, dt,
                                      stream));
@@ -274,15 +297,47 @@ extern "C" int kvr_decoder_layer(const kvr_layer_desc* L, const kvr_refresh_desc
     return KVR_OK;
 }
 
-extern "C" int kvr_decoder_forward(const kvr_layer_desc* layers, int32_t n_layers, const kvr_refresh_desc* d,
-                                   void* hidden, void* stream) {
+int decoder_forward(const kvr_layer_desc* layers, int32_t n_layers, const kvr_refresh_desc* d, void* hidden,
+                    void* stream, bool tiled) {
     if (n_layers < 0) return KVR_E_INVALID_ARGUMENT;
     if (n_layers > 0 && !layers) return KVR_E_NULL_POINTER;
+    const int64_t gemm_need = n_layers > 0 ? gemm_workspace_bytes(d, tiled) : 0;
     for (int32_t i = 0; i < n_layers; ++i) {
-        const int st = kvr_decoder_layer(layers + i, d, hidden, stream);
+        const int st = decoder_layer(layers + i, d, hidden, stream, tiled, gemm_need);
         if (st < 0) return st;
     }
     return KVR_OK;
+}
+
+}  // namespace
+}  // namespace kvr
+
+using namespace kvr;
+
+extern "C" int64_t kvr_decoder_scratch_bytes(const kvr_refresh_desc* d) { return scratch_bytes(d, false); }
+
+extern "C" int64_t kvr_decoder_gemm_workspace_bytes(const kvr_refresh_desc* d) {
+    return gemm_workspace_bytes(d, false);
+}
+
+extern "C" int kvr_decoder_layer(const kvr_layer_desc* L, const kvr_refresh_desc* d, void* hidden, void* stream) {
+    return decoder_layer(L, d, hidden, stream, false, gemm_workspace_bytes(d, false));
+}
+
+extern "C" int kvr_decoder_forward(const kvr_layer_desc* layers, int32_t n_layers, const kvr_refresh_desc* d,
+                                   void* hidden, void* stream) {
+    return decoder_forward(layers, n_layers, d, hidden, stream, false);
+}
+
+extern "C" int64_t kvr_decoder_tiled_scratch_bytes(const kvr_refresh_desc* d) { return scratch_bytes(d, true); }
+
+extern "C" int64_t kvr_decoder_tiled_gemm_workspace_bytes(const kvr_refresh_desc* d) {
+    return gemm_workspace_bytes(d, true);
+}
+
+extern "C" int kvr_decoder_tiled_forward(const kvr_layer_desc* layers, int32_t n_layers, const kvr_refresh_desc* d,
+                                         void* hidden, void* stream) {
+    return decoder_forward(layers, n_layers, d, hidden, stream, true);
 }
 
 extern "C" int kvr_linear_multi_partials(const void* x, int32_t n_weights, const void* const* w,

@@ -359,7 +359,7 @@ int rope_scatter_impl(const void* q, void* q_out, const void* fresh_k, const voi
     if (n_sel == 0) return KVR_OK;
     if (partial) {
         if (!partial->base || partial->splits < 1 || !part_col) return KVR_E_NULL_POINTER;
-        if (dtype_size(dtype) != 2 || n_sel > kPartialTileRows) return KVR_E_UNSUPPORTED_SHAPE;
+        if (dtype_size(dtype) != 2 || n_sel > partial->rows) return KVR_E_UNSUPPORTED_SHAPE;
     } else if (!q || !fresh_k || !fresh_v) {
         return KVR_E_NULL_POINTER;
     }

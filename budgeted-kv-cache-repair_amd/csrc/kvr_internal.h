@@ -4,7 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include "kvrepair.h"
+#include "kvrepair_tiled.h"
 
 namespace kvr {
 
@@ -68,18 +68,29 @@ __device__ inline float silu_gate(float g, float u) {
     return act * u;
 }
 
-// Split-K partial tiles left by linear_multi(..., reduce = false): fp32
-// [ceil(cols / 64)][splits][64 rows][64 cols]; element (row, col) of the
-// projection is the sum over s of tile(col / 64)[s][row][col % 64], added in
+// Split-K partial tiles left by linear_multi / tiled_linear(..., reduce =
+// false): fp32 [ceil(cols / 64)][splits][rows][64 cols]; element (row, col) of
+// the projection is the sum over s of tile(col / 64)[s][row][col % 64], added in
 // split order and rounded to the dtype -- exactly what the reduce kernel writes.
+constexpr int kPartialTileCols = 64;
+constexpr int kPartialTileRows = 64;  // rows of linear_multi's tiles; tiled_linear's have the call's m
 struct PartialSums {
     const float* base = nullptr;  // nullptr: read the dtype tensor instead
     int32_t splits = 0;
+    int32_t rows = kPartialTileRows;
 };
-constexpr int kPartialTileCols = 64;
-constexpr int kPartialTileRows = 64;
 
 int linear_multi(const void* x, int32_t n_weights, const void* const* w, const int32_t* rows, const int64_t* ldw,
+                 void* y, int32_t m, int32_t k, int64_t ldx, int64_t ldy, int32_t epilogue, const void* residual,
+                 int64_t ldr, void* workspace, int64_t workspace_bytes, int32_t dtype, void* stream, bool reduce,
+                 int32_t* splits_out);
+
+// The same projections for more rows (kvr_gemm_tiled.hip): k a multiple of 64,
+// each weight's rows a multiple of 8.
+constexpr int32_t kTiledMaxRows = 1 << 20;
+bool tiled_linear_ok(int32_t m, int32_t rows, int32_t k);
+int64_t tiled_workspace_bytes(int32_t m, int32_t rows, int32_t k);
+int tiled_linear(const void* x, int32_t n_weights, const void* const* w, const int32_t* rows, const int64_t* ldw,
                  void* y, int32_t m, int32_t k, int64_t ldx, int64_t ldy, int32_t epilogue, const void* residual,
                  int64_t ldr, void* workspace, int64_t workspace_bytes, int32_t dtype, void* stream, bool reduce,
                  int32_t* splits_out);
@@ -93,8 +104,8 @@ constexpr int kPartialBatch = 8;
 __device__ inline void partial_sum8(const PartialSums& p, int64_t row, int64_t col, float out[8]) {
     typedef float f32x4_t __attribute__((ext_vector_type(4)));
     const int64_t tile = col / kPartialTileCols;
-    const float* at = p.base + (tile * p.splits * kPartialTileRows + row) * kPartialTileCols + col % kPartialTileCols;
-    const int64_t step = static_cast<int64_t>(kPartialTileRows) * kPartialTileCols;
+    const float* at = p.base + (tile * p.splits * p.rows + row) * kPartialTileCols + col % kPartialTileCols;
+    const int64_t step = static_cast<int64_t>(p.rows) * kPartialTileCols;
     f32x4_t lo = *reinterpret_cast<const f32x4_t*>(at);
     f32x4_t hi = *reinterpret_cast<const f32x4_t*>(at + 4);
     for (int s0 = 1; s0 < p.splits; s0 += kPartialBatch) {
@@ -123,8 +134,8 @@ __device__ inline void partial_sum8(const PartialSums& p, int64_t row, int64_t c
 // One column of `row` summed over the splits in order (fp32, not yet rounded).
 __device__ inline float partial_sum1(const PartialSums& p, int64_t row, int64_t col) {
     const int64_t tile = col / kPartialTileCols;
-    const float* at = p.base + (tile * p.splits * kPartialTileRows + row) * kPartialTileCols + col % kPartialTileCols;
-    const int64_t step = static_cast<int64_t>(kPartialTileRows) * kPartialTileCols;
+    const float* at = p.base + (tile * p.splits * p.rows + row) * kPartialTileCols + col % kPartialTileCols;
+    const int64_t step = static_cast<int64_t>(p.rows) * kPartialTileCols;
     float sum = at[0];
     for (int s0 = 1; s0 < p.splits; s0 += kPartialBatch) {
         float v[kPartialBatch];

@@ -330,7 +330,7 @@ int rms_norm_partials(const PartialSums& x, const void* residual, void* residual
                       void* stream) {
     if (!rms_norm_partials_ok(hidden, dtype)) return KVR_E_UNSUPPORTED_SHAPE;
     if (!x.base || x.splits < 1 || !out || !weight || (residual && !residual_out)) return KVR_E_NULL_POINTER;
-    if (rows <= 0 || rows > kPartialTileRows) return KVR_E_UNSUPPORTED_SHAPE;
+    if (rows <= 0 || rows > x.rows) return KVR_E_UNSUPPORTED_SHAPE;
     NormArgs a;
     a.x = nullptr;
     a.residual = static_cast<const char*>(residual);

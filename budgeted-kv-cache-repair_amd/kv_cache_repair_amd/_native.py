@@ -106,6 +106,10 @@ def _declare(lib: ctypes.CDLL) -> None:
                                               ctypes.c_int32, ctypes.c_int64, ctypes.c_int64, _vp, ctypes.c_int64,
                                               ctypes.c_int32, _vp, _i32p]
     lib.kvr_linear_multi_partials.restype = ctypes.c_int
+    lib.kvr_tiled_linear_workspace_bytes.argtypes = [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32]
+    lib.kvr_tiled_linear_workspace_bytes.restype = ctypes.c_int64
+    lib.kvr_tiled_linear_multi.argtypes = lib.kvr_linear_multi.argtypes
+    lib.kvr_tiled_linear_multi.restype = ctypes.c_int
     lib.kvr_copy_kv_interval.argtypes = [_vp, _vp, _vp, _vp, ctypes.c_int32, ctypes.c_int32, ctypes.c_int64,
                                          ctypes.c_int32, ctypes.c_int64, ctypes.c_int64, _i64p, ctypes.c_int32, _vp]
     lib.kvr_copy_kv_interval.restype = ctypes.c_int
@@ -126,6 +130,12 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.kvr_decoder_layer.restype = ctypes.c_int
     lib.kvr_decoder_forward.argtypes = [_desc_p, ctypes.c_int32, _refresh_p, _vp, _vp]
     lib.kvr_decoder_forward.restype = ctypes.c_int
+    lib.kvr_decoder_tiled_scratch_bytes.argtypes = [_refresh_p]
+    lib.kvr_decoder_tiled_scratch_bytes.restype = ctypes.c_int64
+    lib.kvr_decoder_tiled_gemm_workspace_bytes.argtypes = [_refresh_p]
+    lib.kvr_decoder_tiled_gemm_workspace_bytes.restype = ctypes.c_int64
+    lib.kvr_decoder_tiled_forward.argtypes = [_desc_p, ctypes.c_int32, _refresh_p, _vp, _vp]
+    lib.kvr_decoder_tiled_forward.restype = ctypes.c_int
     lib.kvr_decoder_desc_sizes.argtypes = [_i64p]
     lib.kvr_decoder_desc_sizes.restype = None
     lib.kvr_attention_schedule.argtypes = [_i64p, ctypes.c_int64, ctypes.c_int64, ctypes.c_int32, ctypes.c_int32,
