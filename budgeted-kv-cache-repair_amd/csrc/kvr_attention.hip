@@ -7,8 +7,8 @@
 //
 // Work decomposition (host schedule, kvr_attention_schedule):
 //   selected rows are cut into groups of 64 (four tiles of 16 rows) -- or, when
-//   so few rows would fill under half the grid, into 16-row groups for the
-//   split-key tile kernel below; group g needs keys
+//   so few rows would fill under half the grid, into 16- or 32-row groups where
+//   the schedule's model says that is faster; group g needs keys
 //   [0, pos[last row of g] + 1). That key range is cut into chunks
 //   whose boundaries are multiples of 64 keys, sized so every chunk carries
 //   about the same cost (64-key sub-tiles weighted by how many of the group's
@@ -43,17 +43,12 @@ constexpr int kWorkInts = 4;               // (group, chunk, key_begin, key_end)
 constexpr int kRowTile = 16;               // rows per MFMA tile
 constexpr int kTilesPerGroup = 4;
 constexpr int kGroupRows = kRowTile * kTilesPerGroup;  // rows per group of the wide kernels
-constexpr int kTileGroupRows = kRowTile;               // rows per group of the split-key tile kernel
+constexpr int kHalfGroupRows = 2 * kRowTile;           // ... of the head-pair kernel
+constexpr int kTileGroupRows = kRowTile;               // ... of the head-pair and split-key tile kernels
 constexpr int kSub = 64;                   // keys per LDS sub-tile
 constexpr int kMaxChunksPerGroup = 1024;   // merge weights fit in LDS
 #ifndef KVR_ATTN_TARGET_BLOCKS
 #define KVR_ATTN_TARGET_BLOCKS 256
-#endif
-#ifndef KVR_ATTN_MAX_QT
-#define KVR_ATTN_MAX_QT 4
-#endif
-#ifndef KVR_ATTN_PAIR
-#define KVR_ATTN_PAIR 1
 #endif
 constexpr int kTargetBlocks = KVR_ATTN_TARGET_BLOCKS;  // one block per CU (MI355X: 256 CUs)
 constexpr float kLazyLog2 = 8.f;           // lazy-rescale headroom (log2 units): p <= 256
@@ -738,17 +733,22 @@ __global__ void __launch_bounds__(128 * QT) attn_tile_kernel(AttnArgs a) {
 }
 
 // ===========================================================================
-// Head-pair kernel (bf16 / fp16, head_dim 64 or 128, four query heads per KV
-// head group). Block = (KV head, head group, row group of RT row tiles,
-// chunk), 8 waves. A wave owns two query heads of one 16-row tile -- the two
-// MFMA column tiles share every K and V fragment it reads from LDS, so one
-// fragment read feeds two MFMAs -- and one of X = 8 / (2 RT) key classes.
+// Head-pair kernel (bf16 / fp16, head_dim 64 or 128, a head group of HP = 2 or
+// 1 pairs of query heads on one KV head). Block = (KV head, head group, row
+// group of RT row tiles, chunk), 8 waves. A wave owns two query heads of one
+// 16-row tile -- the two MFMA column tiles share every K and V fragment it
+// reads from LDS, so one fragment read feeds two MFMAs -- and one of
+// X = 8 / (HP RT) key classes.
 // Keys are staged 128 per step (four 32-key sub-tiles) by direct global->LDS
 // loads (no register staging), double-buffered; the wave of key class x
 // attends the step's sub-tiles x, x + X, ... With RT = 1 (16-row groups, few
 // selected rows) the four key classes of a head pair take one sub-tile each
 // per step and are combined through LDS at the end; with RT = 4 (64-row
-// groups) every wave takes all four sub-tiles of a step.
+// groups) every wave takes all four sub-tiles of a step. One pair (HP = 1)
+// runs groups of 32 rows in four classes and of 64 rows in two: against the
+// split-key and wide kernels, which it replaces there but for the fewest rows,
+// 805 rows over 16k keys by 16/8 heads of 64 take 103 us instead of 217, of
+// 128 134 us instead of 499.
 //
 // LDS holds K and V row-major, 16-byte pieces XOR-swizzled by row (piece c of
 // key row r at c ^ (r mod D/8)), so every fragment read below is free of bank
@@ -1300,18 +1300,19 @@ struct PairWave {
     }
 };
 
-template <typename T, int D, int RT, bool HILO>
+template <typename T, int D, int HP, int RT, bool HILO>
 __device__ inline void pair_finish(const AttnArgs& a, PairWave<T, D, HILO>& w, char* smem, int hp, int rt, int kq,
                                    int lane, int lq, int lj, int work, int n_chunks, int head0, int64_t row0,
                                    int32_t kmax, int32_t key_begin);
 
-template <typename T, int D, int RT, bool HILO>
+template <typename T, int D, int HP, int RT, bool HILO>
 __global__ void __launch_bounds__(kPairThreads) attn_pair_kernel(AttnArgs a) {
     using C = PairCfg<D>;
     using W = PairWave<T, D, HILO>;
     using v8 = typename W::v8;
-    constexpr int X = 8 / (2 * RT);  // key classes per head pair
+    constexpr int X = 8 / (HP * RT);  // key classes per head pair
     constexpr int GR = kRowTile * RT;
+    static_assert(X >= 1 && X <= kPairSubs, "every class has a sub-tile of a step");
     extern __shared__ __align__(16) char smem[];
 
     const int tid = threadIdx.x;
@@ -1319,9 +1320,9 @@ __global__ void __launch_bounds__(kPairThreads) attn_pair_kernel(AttnArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lq = lane & 15;
     const int lj = lane >> 4;
-    const int hp = wave & 1;              // head pair of the block's four query heads
-    const int rt = (wave >> 1) % RT;      // row tile within the group
-    const int kq = (wave >> 1) / RT;      // key class
+    const int hp = wave % HP;             // head pair of the block's 2 HP query heads
+    const int rt = (wave / HP) % RT;      // row tile within the group
+    const int kq = (wave / HP) / RT;      // key class
 
     const int work = blockIdx.y;
     const int32_t* wk = work_table_of(a) + kWorkInts * work;
@@ -1331,7 +1332,7 @@ __global__ void __launch_bounds__(kPairThreads) attn_pair_kernel(AttnArgs a) {
     const int n_chunks = group_table(a.sched)[2 * grp + 1];
     const int kv_head = blockIdx.x / a.n_head_groups;
     const int hg = blockIdx.x - kv_head * a.n_head_groups;
-    const int head0 = kv_head * a.group + hg * 4 + 2 * hp;
+    const int head0 = kv_head * a.group + hg * (2 * HP) + 2 * hp;
     const int64_t row0 = static_cast<int64_t>(grp) * GR + kRowTile * rt;
 
     const char* kbase = a.k + (static_cast<int64_t>(kv_head) * a.ks[0] + static_cast<int64_t>(key_begin) * a.ks[1]) * 2;
@@ -1437,16 +1438,16 @@ __global__ void __launch_bounds__(kPairThreads) attn_pair_kernel(AttnArgs a) {
             }
         }
     }
-    pair_finish<T, D, RT, HILO>(a, w, smem, hp, rt, kq, lane, lq, lj, work, n_chunks, head0, row0, kmax, key_begin);
+    pair_finish<T, D, HP, RT, HILO>(a, w, smem, hp, rt, kq, lane, lq, lj, work, n_chunks, head0, row0, kmax, key_begin);
 }
 
 // LDS bytes of pair_finish's exchange: per (head pair, row tile), class and
 // head the D / 16 - D / 16 / X d tiles the class does not own (64 lanes x 16
 // bytes each), then (m, l) per class, head and lane.
-__host__ __device__ constexpr size_t pair_exchange_bytes(int D, int RT) {
-    return RT == 4 ? 0
-                   : static_cast<size_t>(2 * RT) * (8 / (2 * RT)) * 2 *
-                         ((D / 16 - D / 16 / (8 / (2 * RT))) * 64 * 16 + 64 * 8);
+__host__ __device__ constexpr size_t pair_exchange_bytes(int D, int HP, int RT) {
+    return HP * RT == 8 ? 0
+                        : static_cast<size_t>(8) * 2 *
+                              ((D / 16 - D / 16 / (8 / (HP * RT))) * 64 * 16 + 64 * 8);
 }
 
 // Row sums, the combine of the key classes of each (head pair, row tile)
@@ -1456,12 +1457,12 @@ __host__ __device__ constexpr size_t pair_exchange_bytes(int D, int RT) {
 // [SL kq, SL (kq + 1)) of all X classes' O, so the combine's LDS reads and the
 // stores are spread over every wave: each wave first puts its (m, l) and the
 // d tiles it does not own into LDS (f32x4 per lane and tile).
-template <typename T, int D, int RT, bool HILO>
+template <typename T, int D, int HP, int RT, bool HILO>
 __device__ inline void pair_finish(const AttnArgs& a, PairWave<T, D, HILO>& w, char* smem, int hp, int rt, int kq,
                                    int lane, int lq, int lj, int work, int n_chunks, int head0, int64_t row0,
                                    int32_t kmax, int32_t key_begin) {
     using W = PairWave<T, D, HILO>;
-    constexpr int X = 8 / (2 * RT);  // key classes per head pair
+    constexpr int X = 8 / (HP * RT);  // key classes per head pair
     constexpr int GR = kRowTile * RT;
     constexpr int SL = W::DT / X;    // d tiles each wave writes
     static_assert(SL * X == W::DT, "d tiles split evenly over the key classes");
@@ -1490,7 +1491,7 @@ __device__ inline void pair_finish(const AttnArgs& a, PairWave<T, D, HILO>& w, c
         constexpr int kTiles = W::DT - SL;
         const int unit = hp * RT + rt;
         f32x4* xo = reinterpret_cast<f32x4*>(smem);
-        float2* xml = reinterpret_cast<float2*>(smem + static_cast<size_t>(2 * RT) * X * 2 * kTiles * 64 * 16);
+        float2* xml = reinterpret_cast<float2*>(smem + static_cast<size_t>(HP * RT) * X * 2 * kTiles * 64 * 16);
         auto o_at = [&](int c, int t, int dt) {  // dt not owned by class c
             const int k = dt < SL * c ? dt : dt - SL;
             return xo + ((((unit * X + c) * 2 + t) * kTiles + k) * 64 + lane);
@@ -1947,8 +1948,8 @@ __global__ void __launch_bounds__(kFlatThreads) attn_merge_flat_kernel(AttnArgs 
 // Host helpers
 // ---------------------------------------------------------------------------
 int pick_qt(int group) {
-    if (group % 4 == 0 && KVR_ATTN_MAX_QT >= 4) return 4;
-    if (group % 2 == 0 && KVR_ATTN_MAX_QT >= 2) return 2;
+    if (group % 4 == 0) return 4;
+    if (group % 2 == 0) return 2;
     return 1;
 }
 
@@ -1992,34 +1993,36 @@ int launch_tile_inst(const AttnArgs& a, dim3 grid, hipStream_t s) {
     return launch_status();
 }
 
-template <typename T, int D, int RT, bool HILO>
+template <typename T, int D, int HP, int RT, bool HILO>
 int launch_pair_inst(const AttnArgs& a, dim3 grid, hipStream_t s) {
     constexpr size_t bytes = PairCfg<D>::bytes;
-    static_assert(bytes >= pair_exchange_bytes(D, RT), "key-class exchange fits the stages");
-    static const bool ok = allow_lds(attn_pair_kernel<T, D, RT, HILO>, bytes);
+    static_assert(bytes >= pair_exchange_bytes(D, HP, RT), "key-class exchange fits the stages");
+    static const bool ok = allow_lds(attn_pair_kernel<T, D, HP, RT, HILO>, bytes);
     if (!ok) return KVR_E_LAUNCH_FAILED;
-    attn_pair_kernel<T, D, RT, HILO><<<grid, kPairThreads, bytes, s>>>(a);
+    attn_pair_kernel<T, D, HP, RT, HILO><<<grid, kPairThreads, bytes, s>>>(a);
     return launch_status();
+}
+
+template <typename T, int D, int HP, bool HILO>
+int launch_pair(const AttnArgs& a, dim3 grid, hipStream_t s) {
+    if (a.group_rows == kGroupRows) return launch_pair_inst<T, D, HP, 4, HILO>(a, grid, s);
+    if constexpr (HP == 2) {
+        if (a.group_rows == kTileGroupRows) return launch_pair_inst<T, D, HP, 1, HILO>(a, grid, s);
+    } else {
+        if (a.group_rows == kHalfGroupRows) return launch_pair_inst<T, D, HP, 2, HILO>(a, grid, s);
+    }
+    return KVR_E_BAD_SCHEDULE;
 }
 
 template <typename T, int D>
 int launch_mfma(const AttnArgs& a, int qt, dim3 grid, hipStream_t s) {
-    if (qt == 4 && KVR_ATTN_PAIR) {
-        if (a.p_rounded) {
-            if (a.group_rows == kTileGroupRows) return launch_pair_inst<T, D, 1, false>(a, grid, s);
-            return launch_pair_inst<T, D, 4, false>(a, grid, s);
-        }
-        if (a.group_rows == kTileGroupRows) return launch_pair_inst<T, D, 1, true>(a, grid, s);
-        return launch_pair_inst<T, D, 4, true>(a, grid, s);
-    }
-    if (a.group_rows == kTileGroupRows) {
-        if (qt == 4) return launch_tile_inst<T, D, 4>(a, grid, s);
-        if (qt == 2) return launch_tile_inst<T, D, 2>(a, grid, s);
-        return launch_tile_inst<T, D, 1>(a, grid, s);
-    }
-    if (qt == 4) return launch_mfma_inst<T, D, 4>(a, grid, s);
-    if (qt == 2) return launch_mfma_inst<T, D, 2>(a, grid, s);
-    return launch_mfma_inst<T, D, 1>(a, grid, s);
+    if (qt == 4) return a.p_rounded ? launch_pair<T, D, 2, false>(a, grid, s) : launch_pair<T, D, 2, true>(a, grid, s);
+    // two heads: probabilities always as hi + lo (the permission to round them is not used)
+    if (qt == 2)
+        return a.group_rows == kTileGroupRows ? launch_tile_inst<T, D, 2>(a, grid, s) : launch_pair<T, D, 1, true>(a, grid, s);
+    if (a.group_rows == kTileGroupRows) return launch_tile_inst<T, D, 1>(a, grid, s);
+    if (a.group_rows == kGroupRows) return launch_mfma_inst<T, D, 1>(a, grid, s);
+    return KVR_E_BAD_SCHEDULE;
 }
 
 template <typename T, int DMAX>
@@ -2122,11 +2125,17 @@ struct Chunk {
 constexpr int64_t kCostBlock = 16;
 constexpr int64_t kCostMergeChunk = 2;
 
-int64_t chunk_cost(const GroupKeys& k, const Chunk& c) {
-    int64_t cost = 0;
-    for (int64_t s = c.begin / kSub; s < (c.end + kSub - 1) / kSub; ++s) cost += subtile_cost(k, s);
+// Cost of sub-tiles [begin, end) of a group.
+int64_t range_cost(const GroupKeys& k, int64_t begin, int64_t end) {
+    int64_t cost = kCostStage * (end - begin);
+    for (int t = 0; t < kTilesPerGroup; ++t) {
+        const int64_t attended = std::min<int64_t>((k.tile_kmax[t] + kSub - 1) / kSub, end);
+        cost += attended > begin ? kCostTile * (attended - begin) : 0;
+    }
     return cost;
 }
+
+int64_t chunk_cost(const GroupKeys& k, const Chunk& c) { return range_cost(k, c.begin / kSub, (c.end + kSub - 1) / kSub); }
 
 // Longest-first order: whole groups (their chunks stay contiguous and in chunk
 // order, as the merge reads them) sorted by their chunks' largest cost, so the
@@ -2155,6 +2164,53 @@ int64_t schedule_span(const std::vector<GroupKeys>& keys, std::vector<Chunk>& ch
     int64_t merge = 0;
     for (int32_t n : count) merge += n > 1 ? n * kCostMergeChunk : 0;
     return *std::max_element(load.begin(), load.end()) + merge;
+}
+
+// Modelled time (us) of a schedule of the small-row launches, for the choice of
+// the group size: per 128-key step and block of each kernel, its fixed part,
+// 0.3 us per MB of partials and a merge launch of 3 us plus 0.2 us per chunk of
+// its longest chain. Fitted to 210 measured launches (16 to 2048 rows over 2k
+// to 32k keys; 32/8 and 16/4 heads by 4, 16/8 and 8/4 by 2; head dims 64 and
+// 128): the choice costs 0.2% over the fastest group size on average. Where it
+// leaves the 16-row groups: four heads, 400 rows over 16k keys 150 -> 89 us,
+// 805 over 32k 478 -> 297 us; two heads, 282 rows over 8k keys 95 -> 38 us.
+struct StepTimes {
+    double step, block, fixed;
+};
+
+StepTimes step_times(int qt, int head_dim, int group_rows) {
+    const bool wide = head_dim == 128;
+    if (qt == 4) {
+        // between the times with rounded (1.25, 2.82 at head dim 128) and hi + lo
+        // probabilities (1.53, 3.87): the schedule does not depend on that
+        if (group_rows == kTileGroupRows) return {wide ? 1.39 : 0.92, 5.0, 0.0};
+        return {wide ? 3.25 : 2.4, 3.0, 1.0};
+    }
+    if (group_rows == kTileGroupRows) return {wide ? 2.69 : 1.31, 3.0, 0.0};  // split-key tile kernel
+    if (group_rows == kHalfGroupRows) return {wide ? 1.55 : 1.15, 5.0, 2.0};
+    return {wide ? 2.72 : 2.23, 3.0, 2.0};
+}
+
+int64_t partial_bytes(const std::vector<Chunk>& chunks, int64_t n_groups, int32_t n_q_heads, int group_rows,
+                      int32_t head_dim) {
+    if (static_cast<int64_t>(chunks.size()) == n_groups) return 0;  // every group has one chunk
+    return static_cast<int64_t>(n_q_heads) * chunks.size() * group_rows * (head_dim + 2) * 4;
+}
+
+// Each block goes to the CU (of the `cus` of its head's XCD) that frees first.
+double schedule_us(const std::vector<Chunk>& chunks, int64_t n_groups, int64_t cus, const StepTimes& t,
+                   int64_t partials) {
+    std::vector<double> load(static_cast<size_t>(cus), 0.0);
+    std::vector<int32_t> count(static_cast<size_t>(n_groups), 0);
+    int32_t chain = 0;
+    for (const Chunk& c : chunks) {
+        auto least = std::min_element(load.begin(), load.end());
+        *least += ceil_div(c.end - c.begin, 2 * kSub) * t.step + t.block;
+        chain = std::max(chain, ++count[c.group]);
+    }
+    double us = *std::max_element(load.begin(), load.end()) + t.fixed;
+    if (partials > 0) us += partials * 0.3e-6 + 3.0 + 0.2 * chain;
+    return us;
 }
 
 // ---------------------------------------------------------------------------
@@ -2272,13 +2328,15 @@ extern "C" int64_t kvr_attention_schedule_ex(const int64_t* positions, int64_t n
     const int qt = pick_qt(group);
     const int n_head_groups = group / qt;
     const int64_t heads = static_cast<int64_t>(n_kv_heads) * n_head_groups;
-    // Few rows (64-row groups x heads fill under half the grid): 16-row groups
-    // for the split-key tile kernel, so a group needs 4x fewer key chunks for
-    // the same grid and writes 4x less partial data; the chunk's K/V is then
-    // read by up to 4 row groups, from the L2 of the head's XCD.
+    // Few rows (64-row groups x heads fill under half the grid): smaller groups
+    // need fewer key chunks each for the same grid and write less partial data;
+    // larger ones do more matrix work per K/V step (a step of 16 rows takes 0.3
+    // to 0.6 of the time of one of 64). Which wins depends on rows, keys and
+    // heads, so the schedules are compared by modelled time (schedule_us).
     const int64_t wide_units = (n_sel + kGroupRows - 1) / kGroupRows * heads;
-    const int group_rows = (mfma && 2 * wide_units <= kTargetBlocks) ? kTileGroupRows : kGroupRows;
-    const int64_t n_groups = (n_sel + group_rows - 1) / group_rows;
+    const bool few = mfma && 2 * wide_units <= kTargetBlocks;
+    int group_rows = few ? kTileGroupRows : kGroupRows;
+    int64_t n_groups = (n_sel + group_rows - 1) / group_rows;
     if (n_groups == 0) {
         // No selected rows: a header-only schedule (no groups, no work).
         const int64_t need = kHeader;
@@ -2300,49 +2358,31 @@ extern "C" int64_t kvr_attention_schedule_ex(const int64_t* positions, int64_t n
         return need;
     }
 
-    std::vector<GroupKeys> keys(static_cast<size_t>(n_groups));
-    for (int64_t g = 0; g < n_groups; ++g) keys[g] = group_keys(positions, n_sel, g, group_rows);
-
-    std::vector<Chunk> chunks;
-    if (chunk_keys > 0) {
-        // Fixed chunk length (grown by 64 keys while a group would need more
-        // chunks than the merge can weigh).
-        int64_t kc = chunk_keys;
-        for (;;) {
-            int64_t worst = 0;
-            for (int64_t g = 0; g < n_groups; ++g) {
-                const int64_t c = (keys[g].kmax + kc - 1) / kc;
-                worst = c > worst ? c : worst;
-            }
-            if (worst <= kMaxChunksPerGroup) break;
-            kc += kSub;
-        }
-        for (int64_t g = 0; g < n_groups; ++g) {
-            const int64_t c = (keys[g].kmax + kc - 1) / kc;
-            for (int64_t i = 0; i < c; ++i) {
-                const int64_t end = (i + 1) * kc < keys[g].kmax ? (i + 1) * kc : keys[g].kmax;
-                chunks.push_back({static_cast<int32_t>(g), static_cast<int32_t>(i), static_cast<int32_t>(i * kc),
-                                  static_cast<int32_t>(end)});
-            }
-        }
-    } else {
+    std::vector<GroupKeys> keys;
+    auto set_groups = [&](int rows) {
+        group_rows = rows;
+        n_groups = (n_sel + rows - 1) / rows;
+        keys.resize(static_cast<size_t>(n_groups));
+        for (int64_t g = 0; g < n_groups; ++g) keys[g] = group_keys(positions, n_sel, g, rows);
+    };
+    // Cost-balanced chunks of the current groups.
+    auto balanced = [&]() {
         // Cost-balanced chunks: about kTargetBlocks blocks over the whole grid;
         // a group whose cost fits one block's share is not split (no merge).
         int64_t total = 0;
         std::vector<int64_t> group_cost(static_cast<size_t>(n_groups), 0);
         for (int64_t g = 0; g < n_groups; ++g) {
-            const int64_t n_sub = (keys[g].kmax + kSub - 1) / kSub;
-            for (int64_t s = 0; s < n_sub; ++s) group_cost[g] += subtile_cost(keys[g], s);
+            group_cost[g] = range_cost(keys[g], 0, (keys[g].kmax + kSub - 1) / kSub);
             total += group_cost[g];
         }
         const int64_t per_head = kTargetBlocks / heads > 1 ? kTargetBlocks / heads : 1;
         const int64_t max_cost = *std::max_element(group_cost.begin(), group_cost.end());
         // (The head-pair kernel also runs one block per CU in 64-row groups.)
-        const bool one_block_per_cu = group_rows == kTileGroupRows || (mfma && qt == 4 && KVR_ATTN_PAIR);
+        const bool one_block_per_cu = group_rows == kTileGroupRows || (mfma && qt >= 2);
         // The head-pair kernel walks a chunk in steps of two sub-tiles from its
         // first key: a boundary after an odd number of sub-tiles would leave a
         // half-empty step, so inner boundaries close on whole steps.
-        const bool pair_steps = mfma && qt == 4 && KVR_ATTN_PAIR && kPairStepKeys == 2 * kSub;
+        const bool pair_steps = mfma && qt >= 2 && kPairStepKeys == 2 * kSub;
         // Chunks for a share of `share` blocks per head.
         auto build = [&](int64_t share) {
             auto chunks_of = [&](int64_t g, int64_t cap) {
@@ -2398,8 +2438,10 @@ extern "C" int64_t kvr_attention_schedule_ex(const int64_t* positions, int64_t n
             }
             return out;
         };
-        chunks = build(per_head);
-        if (group_rows == kGroupRows && one_block_per_cu) {
+        std::vector<Chunk> chunks = build(per_head);
+        // (Of few rows, only where a block's share is long enough, 8 steps, to be cut.)
+        if (group_rows == kGroupRows && one_block_per_cu &&
+            (!few || total > per_head * 16 * (kCostStage + kTilesPerGroup * kCostTile))) {
             // 64-row groups (MFMA-bound launches): one block per CU means one round
             // is balanced only as well as the chunk costs are. Two or four rounds
             // of smaller chunks let the dispatcher even the CUs out; keep the
@@ -2413,6 +2455,60 @@ extern "C" int64_t kvr_attention_schedule_ex(const int64_t* positions, int64_t n
                     chunks = std::move(more);
                 }
             }
+        }
+        return chunks;
+    };
+    set_groups(group_rows);
+    std::vector<Chunk> chunks;
+    if (chunk_keys > 0) {
+        // Fixed chunk length (grown by 64 keys while a group would need more
+        // chunks than the merge can weigh).
+        int64_t kc = chunk_keys;
+        for (;;) {
+            int64_t worst = 0;
+            for (int64_t g = 0; g < n_groups; ++g) {
+                const int64_t c = (keys[g].kmax + kc - 1) / kc;
+                worst = c > worst ? c : worst;
+            }
+            if (worst <= kMaxChunksPerGroup) break;
+            kc += kSub;
+        }
+        for (int64_t g = 0; g < n_groups; ++g) {
+            const int64_t c = (keys[g].kmax + kc - 1) / kc;
+            for (int64_t i = 0; i < c; ++i) {
+                const int64_t end = (i + 1) * kc < keys[g].kmax ? (i + 1) * kc : keys[g].kmax;
+                chunks.push_back({static_cast<int32_t>(g), static_cast<int32_t>(i), static_cast<int32_t>(i * kc),
+                                  static_cast<int32_t>(end)});
+            }
+        }
+    } else {
+        chunks = balanced();
+        if (few && qt >= 2) {
+            const int64_t cus = kTargetBlocks / heads > 1 ? kTargetBlocks / heads : 1;
+            auto rate = [&](const std::vector<Chunk>& c) {
+                return schedule_us(c, n_groups, cus, step_times(qt, head_dim, group_rows),
+                                   partial_bytes(c, n_groups, n_q_heads, group_rows, head_dim));
+            };
+            double least = rate(chunks);
+            std::vector<GroupKeys> best_keys = keys;
+            int best_rows = group_rows;
+            for (int rows : {kHalfGroupRows, kGroupRows}) {
+                if (rows == kHalfGroupRows && qt != 2) continue;  // four heads: never the fastest
+                set_groups(rows);
+                std::vector<Chunk> other = balanced();
+                // what the static scratch of the allocation-free entry point holds, it keeps holding
+                if (partial_bytes(other, n_groups, n_q_heads, group_rows, head_dim) > kScratchBytes) continue;
+                const double us = rate(other);
+                if (us < least) {
+                    least = us;
+                    chunks = std::move(other);
+                    best_keys = keys;
+                    best_rows = rows;
+                }
+            }
+            group_rows = best_rows;
+            n_groups = (n_sel + group_rows - 1) / group_rows;
+            keys = std::move(best_keys);
         }
     }
     const int64_t n_work = static_cast<int64_t>(chunks.size());
@@ -2479,7 +2575,9 @@ extern "C" int64_t kvr_attention_workspace_bytes(const int32_t* schedule, int64_
     if (!schedule || schedule_len < kHeader || schedule[H_MAGIC] != kMagic || schedule[H_VERSION] != kVersion)
         return KVR_E_BAD_SCHEDULE;
     if (schedule[H_HQ] != n_q_heads || schedule[H_D] != head_dim) return KVR_E_BAD_SCHEDULE;
-    if (schedule[H_GROUP_ROWS] != kGroupRows && schedule[H_GROUP_ROWS] != kTileGroupRows) return KVR_E_BAD_SCHEDULE;
+    if (schedule[H_GROUP_ROWS] != kGroupRows && schedule[H_GROUP_ROWS] != kHalfGroupRows &&
+        schedule[H_GROUP_ROWS] != kTileGroupRows)
+        return KVR_E_BAD_SCHEDULE;
     if (schedule[H_NMULTI] == 0) return 0;
     return static_cast<int64_t>(n_q_heads) * schedule[H_NWORK] * schedule[H_GROUP_ROWS] * (head_dim + 2) * 4;
 }

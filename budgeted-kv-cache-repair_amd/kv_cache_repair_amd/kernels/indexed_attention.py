@@ -149,11 +149,18 @@ def _host_schedule(host_plan: "IndexedPlan", key: tuple, positions=None):
     pos = _native.i64_array(host_plan.positions) if positions is None else positions
     args = (pos, host_plan.selected_count, host_plan.logical_length, n_q_heads, n_kv_heads, head_dim,
             _native.DTYPE_CODES[dtype], chunk_keys, _native.ATTN_ROUNDED_PROBABILITIES if rounded else 0)
-    need = lib.kvr_attention_schedule_ex(*args, None, 0)
-    _native.check(int(need), "kvr_attention_schedule_ex")
-    host = (ctypes.c_int32 * int(need))()
-    _native.check(int(lib.kvr_attention_schedule_ex(*args, host, int(need))), "kvr_attention_schedule_ex")
-    return host
+    # room for every schedule chosen from the geometry (at most four rounds of 256
+    # blocks, or one chunk per 16-row group), so it is computed once; a fixed
+    # chunk size may need more and asks first
+    groups = (host_plan.selected_count + 15) // 16
+    room = 18 + 2 * groups + 4 * (1024 + groups)
+    if chunk_keys > 0:
+        room = int(lib.kvr_attention_schedule_ex(*args, None, 0))
+        _native.check(room, "kvr_attention_schedule_ex")
+    host = (ctypes.c_int32 * room)()
+    need = int(lib.kvr_attention_schedule_ex(*args, host, room))
+    _native.check(need, "kvr_attention_schedule_ex")
+    return (ctypes.c_int32 * need).from_buffer_copy(memoryview(host).cast("B")[:4 * need])
 
 
 def _upload(parts, device: torch.device) -> torch.Tensor:
