@@ -27,9 +27,9 @@
 // (no bank conflicts measured).
 //
 // Measured (us; hipBLASLt's separate q, k, v, o, gate, up, down, SiLU and
-// residual launches of one 8B layer in brackets): 71 rows 97 (210), 141 rows
-// 118 (230), 282 rows 161 (270), 512 rows 214 (310), 1383 rows 553 (560). Rates:
-// gate/up at 71 rows 52 us = 4.5 TB/s of weights; 256 x 256 tiles 1.4-1.45
+// residual launches of one 8B layer in brackets): 71 rows 92 (210), 141 rows
+// 112 (230), 282 rows 161 (270), 512 rows 211 (310), 1383 rows 545 (560). Rates:
+// gate/up at 71 rows 42.5 us = 5.5 TB/s of weights; 256 x 256 tiles 1.4-1.45
 // PFLOP/s at 4096 rows (2.05 GHz; 1.72 with the loads left out, so LDS traffic
 // and the issue slots of the loads are what is left).
 #include "kvr_internal.h"
@@ -64,6 +64,7 @@ constexpr int kRowBytes = 128;
 constexpr int kGroupRows = 8;     // rows of one wave-wide 1 KB load
 constexpr int kXcds = 8;
 constexpr int kCusPerXcd = 32;
+constexpr int kStreamRows = 192;  // STREAM tiles
 constexpr int kPanelGroup = 4;    // weight panels that consecutive blocks of an XCD walk together
 
 struct TiledArgs {
@@ -86,9 +87,15 @@ struct TiledArgs {
 };
 
 // 16 bytes per lane from `base` (wave-uniform) + off into LDS at dst
-// (wave-uniform) + 16 * lane.
+// (wave-uniform) + 16 * lane; the second form with the nontemporal hint.
 __device__ inline void load_lds(const char* base, uint32_t off, uint32_t dst) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off),
+                 "s"(reinterpret_cast<uint64_t>(base)), "s"(dst)
+                 : "memory", "m0");
+}
+
+__device__ inline void load_lds_once(const char* base, uint32_t off, uint32_t dst) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off),
                  "s"(reinterpret_cast<uint64_t>(base)), "s"(dst)
                  : "memory", "m0");
 }
@@ -143,7 +150,14 @@ struct TileCfg {
 // read (one piece column) then cover all 64 banks.
 __device__ constexpr int swz(int r) { return (r >> 1) & 7; }
 
-template <typename T, typename C>
+// STREAM (one x tile of at most 192 rows: every weight byte is read once, and
+// reading them is what bounds the launch): weights load nontemporally, and
+// weight panel p starts at stage p of its k range and wraps around, so that
+// concurrent blocks are not all at the same offset of their 8 KB and longer
+// rows. Gate/up of an 8B model, 71 rows: 53.7 us, 49.4 nontemporal, 42.6 with
+// the staggered start too (5.5 TB/s); 160 rows: 61.7, 58.8, 57.2. With more rows
+// per panel or several x tiles, which read a panel together, both lose.
+template <typename T, typename C, bool STREAM>
 __global__ void __launch_bounds__(C::kThreads) tiled_gemm_kernel(TiledArgs a) {
     using G = tile_t<T>;
     using E = elem<T>;
@@ -240,6 +254,26 @@ __global__ void __launch_bounds__(C::kThreads) tiled_gemm_kernel(TiledArgs a) {
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // load l of the stage that comes next (`next_k` its byte offset in the k range) to LDS offset `at`
+    const int64_t k_bytes = static_cast<int64_t>(steps) * kRowBytes;
+    int64_t next_k = STREAM ? static_cast<int64_t>(panel % steps) * kRowBytes : 0;
+    auto load = [&](int l, uint32_t at) __attribute__((always_inline)) {
+        if constexpr (STREAM) {
+            if (wave + l * C::kWaves < BN / kGroupRows)
+                load_lds_once(base[l] + next_k, off[l], dst[l] + at);
+            else
+                load_lds(base[l] + next_k, off[l], dst[l] + at);
+        } else {
+            load_lds(base[l], off[l], dst[l] + at);
+            base[l] += kRowBytes;
+        }
+    };
+    auto loaded = [&]() __attribute__((always_inline)) {
+        if constexpr (STREAM) {
+            next_k += kRowBytes;
+            if (next_k == k_bytes) next_k = 0;
+        }
+    };
     // The MFMAs of half kk, with the reads of the other half's next fragments
     // (and, with_load, the loads of a stage) issued between the first three
     // quarters of them.
@@ -254,8 +288,7 @@ __global__ void __launch_bounds__(C::kThreads) tiled_gemm_kernel(TiledArgs a) {
             if constexpr (decltype(with_load)::value)
                 static_for<l1 - l0>([&](auto lc) __attribute__((always_inline)) {
                     constexpr int l = l0 + decltype(lc)::value;
-                    load_lds(base[l], off[l], dst[l] + load_at);
-                    base[l] += kRowBytes;
+                    load(l, load_at);
                 });
             static_for<f1 - f0>([&](auto fc) __attribute__((always_inline)) {
                 read(kk ^ 1, read_at, f0 + decltype(fc)::value);
@@ -268,10 +301,8 @@ __global__ void __launch_bounds__(C::kThreads) tiled_gemm_kernel(TiledArgs a) {
         constexpr int s = decltype(sc)::value;
         if (s < steps) {
 #pragma unroll
-            for (int l = 0; l < L; ++l) {
-                load_lds(base[l], off[l], dst[l] + s * C::kStage);
-                base[l] += kRowBytes;
-            }
+            for (int l = 0; l < L; ++l) load(l, s * C::kStage);
+            loaded();
         }
     });
     if (steps >= NST)
@@ -296,6 +327,7 @@ __global__ void __launch_bounds__(C::kThreads) tiled_gemm_kernel(TiledArgs a) {
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
         multiply(1, with_load, next, static_cast<uint32_t>(stage));
+        if constexpr (decltype(with_load)::value) loaded();
         stage = next;
     };
     int s = 0;
@@ -416,27 +448,28 @@ __global__ void __launch_bounds__(kReduceThreads) tiled_reduce_kernel(TiledArgs 
 // differ in how many rows they cover with the weights read once and in how
 // they divide a projection's grid into whole rounds of 256 CUs.
 #define KVR_TILES(X) \
-    X(8, 4, 2, 4, 2, 1.40f) /* 256 x 256 */ \
-    X(7, 4, 2, 4, 2, 1.33f) /* 224 x 256 */ \
-    X(6, 4, 2, 4, 2, 1.21f) /* 192 x 256 */ \
-    X(5, 4, 2, 4, 3, 0.96f) /* 160 x 256 */ \
-    X(4, 4, 2, 4, 3, 0.80f) /* 128 x 256 */ \
-    X(6, 3, 3, 4, 2, 1.29f) /* 288 x 192 */ \
-    X(9, 2, 2, 4, 3, 0.89f) /* 288 x 128 */ \
-    X(8, 2, 2, 4, 3, 0.78f) /* 256 x 128 */ \
-    X(7, 2, 2, 4, 3, 0.73f) /* 224 x 128 */ \
-    X(6, 2, 2, 4, 3, 0.62f) /* 192 x 128 */ \
-    X(5, 2, 2, 4, 4, 0.58f) /* 160 x 128 */ \
+    X(8, 4, 2, 4, 2, 1.23f) /* 256 x 256 */ \
+    X(7, 4, 2, 4, 2, 1.23f) /* 224 x 256 */ \
+    X(6, 4, 2, 4, 2, 1.16f) /* 192 x 256 */ \
+    X(5, 4, 2, 4, 3, 0.90f) /* 160 x 256 */ \
+    X(4, 4, 2, 4, 3, 0.81f) /* 128 x 256 */ \
+    X(6, 3, 3, 4, 2, 1.19f) /* 288 x 192 */ \
+    X(9, 2, 2, 4, 3, 0.86f) /* 288 x 128 */ \
+    X(8, 2, 2, 4, 3, 0.77f) /* 256 x 128 */ \
+    X(7, 2, 2, 4, 3, 0.75f) /* 224 x 128 */ \
+    X(6, 2, 2, 4, 3, 0.60f) /* 192 x 128 */ \
+    X(5, 2, 2, 4, 4, 0.60f) /* 160 x 128 */ \
     X(3, 2, 3, 4, 4, 0.52f) /* 144 x 128 */ \
     X(4, 2, 2, 4, 4, 0.46f) /* 128 x 128 */ \
     X(3, 2, 2, 4, 4, 0.43f) /* 96 x 128 */ \
-    X(5, 1, 1, 7, 4, 0.36f) /* 80 x 112 */ \
-    X(6, 1, 1, 7, 4, 0.39f) /* 96 x 112 */ \
+    X(5, 1, 1, 8, 4, 0.37f) /* 80 x 128 */ \
+    X(5, 1, 1, 7, 4, 0.31f) /* 80 x 112 */ \
+    X(6, 1, 1, 7, 4, 0.36f) /* 96 x 112 */ \
     X(9, 1, 1, 7, 4, 0.51f) /* 144 x 112 */ \
-    X(5, 1, 1, 4, 4, 0.23f) /* 80 x 64 */ \
-    X(8, 1, 1, 4, 4, 0.35f) /* 128 x 64 */ \
-    X(5, 1, 1, 6, 4, 0.34f) /* 80 x 96 */ \
-    X(8, 1, 1, 6, 4, 0.44f) /* 128 x 96 */
+    X(5, 1, 1, 4, 4, 0.27f) /* 80 x 64 */ \
+    X(8, 1, 1, 4, 4, 0.41f) /* 128 x 64 */ \
+    X(5, 1, 1, 6, 4, 0.29f) /* 80 x 96 */ \
+    X(8, 1, 1, 6, 4, 0.43f) /* 128 x 96 */
 
 struct Tile {
     int32_t bm, bn;
@@ -458,31 +491,35 @@ struct Choice {
     int32_t split_steps;
 };
 
-// The tile and K split with the least modelled time, of a model fitted to 190
-// measured projections (q/k/v, o, gate/up, down of 8B shapes, 66 to 8192 rows;
-// the choice is 1.3% slower than the fastest tile on average, 14% at most):
-// blocks run in rounds of 32 CUs per XCD, a round costs its stages plus 1.0 us
-// (3.6 us more for the gated epilogue); against it the weight stream, 5.6 TB/s
-// with every CU loading; both overlap as a 2-norm. Split partials cost 0.2
-// us/MB to write and about as much again in their consumer.
+// The tile and K split with the least modelled time, of a model fitted to 260
+// measured projections (q/k/v, o, gate/up, down of 8B shapes, 65 to 8192 rows;
+// the choice is 0.7% slower than the fastest tile on average, 19% at most):
+// blocks run in rounds of 32 CUs per XCD, a round costs its stages plus 2.1 us
+// (2.3 us more for the gated epilogue); against it stands the weight stream,
+// 5.9 TB/s with every CU loading, 7.0 nontemporal; both overlap as a 2-norm.
+// Split partials cost 0.16 us/MB to write and 0.2 in their consumer. The
+// smallest tile has no place beside other x tiles: two of its blocks share a CU.
 Choice model_choice(int32_t m, int32_t rows, int32_t k, bool gated) {
     const int32_t steps = k / kStageK;
     Choice best{0, 1, steps};
     double least = 1e30;
     for (int t = 0; t < kTileCount; ++t) {
         const Tile& tile = kTiles[t];
-        const int64_t tiles = ceil_div(m, tile.bm) * ceil_div(rows, tile.bn);
+        const int64_t tiles_m = ceil_div(m, tile.bm);
+        if (tile.bm == 80 && tile.bn == 64 && tiles_m > 1) continue;
+        const int64_t tiles = tiles_m * ceil_div(rows, tile.bn);
+        const bool once = tiles_m == 1 && tile.bm <= kStreamRows;
         for (int32_t want = 1; want <= kMaxSplits; want *= 2) {
             if (want > 1 && (gated || steps / want < kMinSplitSteps)) break;
             const int32_t split_steps = static_cast<int32_t>(ceil_div(steps, want));
             const int32_t splits = static_cast<int32_t>(ceil_div(steps, split_steps));
             const int64_t blocks = tiles * splits;
             const int64_t rounds = ceil_div(ceil_div(blocks, kXcds), kCusPerXcd);
-            const double work = rounds * (split_steps * static_cast<double>(tile.step_us) + (gated ? 4.6 : 1.0));
+            const double work = rounds * (split_steps * static_cast<double>(tile.step_us) + (gated ? 4.4 : 2.1));
             const double busy = blocks < 256 ? static_cast<double>(blocks) / 256 : 1.0;
-            const double stream = static_cast<double>(rows) * k * 2 / 5.6e6 / sqrt(busy);
+            const double stream = static_cast<double>(rows) * k * 2 / (once ? 7.0e6 : 5.9e6) / sqrt(busy);
             double us = sqrt(work * work + stream * stream);
-            if (splits > 1) us += static_cast<double>(m) * rows * 4 * splits * 0.4e-6;
+            if (splits > 1) us += static_cast<double>(m) * rows * 4 * splits * 0.36e-6;
             if (us < least) {
                 least = us;
                 best = Choice{t, splits, split_steps};
@@ -511,15 +548,24 @@ Choice choose(int32_t m, int32_t rows, int32_t k, bool gated) {
     return c;
 }
 
-template <typename T, typename C>
+template <typename T, typename C, bool STREAM>
 int launch_tile(const TiledArgs& a, hipStream_t s) {
-    static const bool ok =
-        C::kLds <= 65536 || hipFuncSetAttribute(reinterpret_cast<const void*>(tiled_gemm_kernel<T, C>),
-                                                hipFuncAttributeMaxDynamicSharedMemorySize, C::kLds) == hipSuccess;
+    static const bool ok = C::kLds <= 65536 ||
+                           hipFuncSetAttribute(reinterpret_cast<const void*>(tiled_gemm_kernel<T, C, STREAM>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, C::kLds) == hipSuccess;
     if (!ok) return KVR_E_LAUNCH_FAILED;
     const int64_t total = static_cast<int64_t>(a.tiles_m) * a.tiles_n * a.splits;
-    tiled_gemm_kernel<T, C><<<static_cast<unsigned>(ceil_div(total, kXcds) * kXcds), C::kThreads, C::kLds, s>>>(a);
+    tiled_gemm_kernel<T, C, STREAM>
+        <<<static_cast<unsigned>(ceil_div(total, kXcds) * kXcds), C::kThreads, C::kLds, s>>>(a);
     return launch_status();
+}
+
+template <typename T, typename C>
+int launch_tile(const TiledArgs& a, hipStream_t s) {
+    if constexpr (C::BM <= kStreamRows) {
+        if (a.tiles_m == 1) return launch_tile<T, C, true>(a, s);
+    }
+    return launch_tile<T, C, false>(a, s);
 }
 
 template <typename T>
