@@ -36,9 +36,6 @@ namespace {
 #ifndef KVR_GEMM_CHUNK_STEPS
 #define KVR_GEMM_CHUNK_STEPS 8
 #endif
-#ifndef KVR_GEMM_RING_CHUNKS
-#define KVR_GEMM_RING_CHUNKS 1
-#endif
 
 // Waves per block (16 streamed weight rows each) is a launch parameter: 4, 6 or
 // 7, whichever makes the grid exactly one block per CU (plan_split).
@@ -52,8 +49,7 @@ struct WaveCfg {
 constexpr int kRowsMax = 64;                // M <= 64 (four 16-row MFMA tiles)
 constexpr int kStep = 32;                   // K per MFMA
 constexpr int kSliceChunk = KVR_GEMM_CHUNK_STEPS * kStep;  // split-K slices are whole multiples of this
-constexpr int kRingChunks = KVR_GEMM_RING_CHUNKS;  // W ring depth in chunks
-static_assert(kRingChunks == 1 || kRingChunks == 2, "chunk buffers alternate with the ring");
+constexpr int kPhaseRows = 1344;            // a multiple of every tile width: 32, 48, 56 features; 64, 96, 112 rows
 
 // Staged x chunk of CS k-steps (CS = the W ring depth per chunk): 8 for
 // launches of at most one block per CU, 4 (half the LDS, chunks turned over
@@ -64,7 +60,7 @@ struct ChunkCfg {
     static constexpr int kChunk = CS * kStep;         // K per chunk
     static constexpr int kXStride = kChunk + 8;       // LDS row stride (elements): 16 B pad, conflict-free B reads
     static constexpr int kXBuf = kRowsMax * kXStride; // one chunk buffer (elements)
-    static constexpr int kRing = kRingChunks * CS;    // W fragments in flight per lane (k-steps)
+    static constexpr int kRing = CS;                 // W fragments in flight per lane (k-steps)
     static constexpr int kGranules = kChunk / 8;      // 16-B x granules per row per chunk
     static constexpr int kXGranules = kRowsMax * kGranules;  // x granules per chunk
     static constexpr int kXLoads = (kXGranules + 64 * NW - 1) / (64 * NW);  // x granules per thread per chunk (at most)
@@ -211,10 +207,24 @@ skinny_gemm_kernel(GemmArgs a) {
     // transposed to the two MFMA A fragments of k-steps 2u, 2u + 1 through a
     // 2 KB per-wave LDS tile (pieces XOR-swizzled by row: conflict-free).
     const int klast = klen - 8;
+    const int chunks = (klen + kChunk - 1) / kChunk;
+    // Position c of the walk is chunk (first + c) mod chunks of the slice: blocks
+    // kPhaseRows streamed rows (gated: features) apart start kSliceChunk apart,
+    // so that they do not all read at the same offset of their weight rows at
+    // once (gate/up of an 8B model over 37 rows 42.6 -> 39.6 us = 5.9 TB/s; the
+    // 32 layers of a 64-row refresh 4.74 -> 4.52 ms). The start depends on the
+    // rows alone, not on the launch's block width, so a weight sums in the same
+    // order in every launch of the same split.
+    const int first_row = tile * (a.gated ? kHalf : kTileN);
+    const int first = first_row / kPhaseRows % ((klen + kSliceChunk - 1) / kSliceChunk) * (kSliceChunk / kChunk);
+    auto chunk_at = [&](int c) __attribute__((always_inline)) -> int {
+        const int at = first + c;  // c <= chunks: at most one turn
+        return at >= chunks ? at - chunks : at;
+    };
     u32x4 wf[kRing];
     const char* wrow[2] = {row_ptr(lane >> 3), row_ptr(8 + (lane >> 3))};
-    auto load_w = [&](int s, int h) __attribute__((always_inline)) -> u32x4 {
-        const int kk = min((s >> 1) * 64 + 8 * (lane & 7), klast);
+    auto load_w = [&](int chunk, int d, int h) __attribute__((always_inline)) -> u32x4 {
+        const int kk = min(chunk * kChunk + (d >> 1) * 64 + 8 * (lane & 7), klast);
         return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wrow[h] + kk * 2));
     };
     char* wtile = reinterpret_cast<char*>(xs + 2 * kXBuf) + wave * 2048;
@@ -248,11 +258,10 @@ skinny_gemm_kernel(GemmArgs a) {
         }
     };
 
-    const int chunks = (klen + kChunk - 1) / kChunk;
-    load_x(0);
+    load_x(first);
 #pragma unroll
-    for (int d = 0; d < kRing; ++d) wf[d] = load_w(d, d & 1);
-    store_x(0, xs);
+    for (int d = 0; d < kRing; ++d) wf[d] = load_w(first, d, d & 1);
+    store_x(first, xs);
     __syncthreads();
 
     f32x4 acc[MT];
@@ -261,44 +270,39 @@ skinny_gemm_kernel(GemmArgs a) {
 
     // Chunk c: issue chunk c + 1's x loads, multiply chunk c pair by pair
     // (copy the pair's two loads into the transpose tile, refill their slots
-    // with the loads kRing steps ahead, read back the two A fragments, run the
-    // MFMAs), then store chunk c + 1 into the other buffer. The loop advances kRingChunks chunks at a time so every ring slot
-    // index is static; a chunk past the last one multiplies an all-zero x
-    // buffer (store_x zeroes k >= klen) and adds nothing. Past the slice the
-    // loads repeat in-bounds addresses into the idle buffer or unread slots.
+    // with the next chunk's loads, read back the two A fragments, run the
+    // MFMAs), then store chunk c + 1 into the other buffer. After the last chunk
+    // the walk comes round to its first: those loads go into the idle buffer and
+    // unread slots.
     // sched_barrier pins the loads where they are written: left alone, the
     // scheduler sinks them to the end of the chunk and exposes their latency.
-    for (int c = 0; c < chunks; c += kRingChunks) {
+    for (int c = 0; c < chunks; ++c) {
+        const uint16_t* cur = xs + (c & 1) * kXBuf;
+        const int ahead = chunk_at(c + 1);
+        load_x(ahead);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int r = 0; r < kRingChunks; ++r) {
-            const int cc = c + r;
-            const uint16_t* cur = xs + (cc & 1) * kXBuf;
-            load_x(cc + 1);
-            __builtin_amdgcn_sched_barrier(0);
+        for (int d = 0; d < kChunkSteps; d += 2) {
+            *reinterpret_cast<u32x4*>(wput) = wf[d];
+            *reinterpret_cast<u32x4*>(wput + 1024) = wf[d + 1];
+            wf[d] = load_w(ahead, d, 0);
+            wf[d + 1] = load_w(ahead, d + 1, 1);
+            const v8 af0 = __builtin_bit_cast(v8, *reinterpret_cast<const u32x4*>(wget0));
+            const v8 af1 = __builtin_bit_cast(v8, *reinterpret_cast<const u32x4*>(wget1));
+            u32x4 bf0[MT], bf1[MT];
 #pragma unroll
-            for (int d = 0; d < kChunkSteps; d += 2) {
-                const int slot = (r * kChunkSteps + d) % kRing;
-                *reinterpret_cast<u32x4*>(wput) = wf[slot];
-                *reinterpret_cast<u32x4*>(wput + 1024) = wf[slot + 1];
-                wf[slot] = load_w(cc * kChunkSteps + d + kRing, 0);
-                wf[slot + 1] = load_w(cc * kChunkSteps + d + 1 + kRing, 1);
-                const v8 af0 = __builtin_bit_cast(v8, *reinterpret_cast<const u32x4*>(wget0));
-                const v8 af1 = __builtin_bit_cast(v8, *reinterpret_cast<const u32x4*>(wget1));
-                u32x4 bf0[MT], bf1[MT];
-#pragma unroll
-                for (int t = 0; t < MT; ++t) {
-                    bf0[t] = *reinterpret_cast<const u32x4*>(cur + (16 * t + lq) * kXStride + d * kStep + 8 * lj);
-                    bf1[t] = *reinterpret_cast<const u32x4*>(cur + (16 * t + lq) * kXStride + (d + 1) * kStep + 8 * lj);
-                }
-#pragma unroll
-                for (int t = 0; t < MT; ++t) acc[t] = G::mma(af0, __builtin_bit_cast(v8, bf0[t]), acc[t]);
-#pragma unroll
-                for (int t = 0; t < MT; ++t) acc[t] = G::mma(af1, __builtin_bit_cast(v8, bf1[t]), acc[t]);
-                __builtin_amdgcn_sched_barrier(0);
+            for (int t = 0; t < MT; ++t) {
+                bf0[t] = *reinterpret_cast<const u32x4*>(cur + (16 * t + lq) * kXStride + d * kStep + 8 * lj);
+                bf1[t] = *reinterpret_cast<const u32x4*>(cur + (16 * t + lq) * kXStride + (d + 1) * kStep + 8 * lj);
             }
-            store_x(cc + 1, xs + ((cc + 1) & 1) * kXBuf);
-            __syncthreads();
+#pragma unroll
+            for (int t = 0; t < MT; ++t) acc[t] = G::mma(af0, __builtin_bit_cast(v8, bf0[t]), acc[t]);
+#pragma unroll
+            for (int t = 0; t < MT; ++t) acc[t] = G::mma(af1, __builtin_bit_cast(v8, bf1[t]), acc[t]);
+            __builtin_amdgcn_sched_barrier(0);
         }
+        store_x(ahead, xs + ((c + 1) & 1) * kXBuf);
+        __syncthreads();
     }
 
     uint16_t* y = reinterpret_cast<uint16_t*>(a.y);
