@@ -213,8 +213,9 @@ skinny_gemm_kernel(GemmArgs a) {
     // so that they do not all read at the same offset of their weight rows at
     // once (gate/up of an 8B model over 37 rows 42.6 -> 39.6 us = 5.9 TB/s; the
     // 32 layers of a 64-row refresh 4.74 -> 4.52 ms). The start depends on the
-    // rows alone, not on the launch's block width, so a weight sums in the same
-    // order in every launch of the same split.
+    // row's place in the launch (gated: the feature's), not on its block width,
+    // so the gated launch sums gate and up in the order of their own launches of
+    // the same split.
     const int first_row = tile * (a.gated ? kHalf : kTileN);
     const int first = first_row / kPhaseRows % ((klen + kSliceChunk - 1) / kSliceChunk) * (kSliceChunk / kChunk);
     auto chunk_at = [&](int c) __attribute__((always_inline)) -> int {

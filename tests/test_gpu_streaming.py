@@ -1,0 +1,49 @@
+"""The streaming projections' staggered walk over k (kvr_linear_multi, at most 64
+rows): tiles 1344 streamed rows apart start at different 256-k chunks of their
+slice and come round, so some start at a last chunk that k leaves ragged."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from test_gpu_operators import assert_linear_close, bits_equal, exact_linear, ulp_distance
+
+# (n, k, splits): one ragged chunk; starts at chunks 0, 1, 2, 0 of three, the last 8, 8 and 248 k long; a slice of
+# two chunks and a ragged second slice; more than 256 blocks (128-k chunks), the last chunk 8 and 248 k long
+SHAPES = [(1400, 200, 1), (5400, 520, 1), (4040, 520, 1), (4100, 760, 1), (6000, 1288, 2), (16400, 520, 1),
+          (17000, 1016, 1)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("rows", [3, 64])
+def test_every_start_of_the_walk_gives_the_product(gpu_device, dtype, shape, rows):
+    from kv_cache_repair_amd import _native
+    from kv_cache_repair_amd.kernels import projection
+
+    n, k, splits = shape
+    assert _native.lib().kvr_linear_splits(rows, n, k) == splits
+    torch.manual_seed(n + k)
+    x = torch.randn(1, rows, k + 8, device=gpu_device).to(dtype)[..., :k]
+    w = (torch.randn(n, k + 8, device=gpu_device) * 0.03).to(dtype)[:, 8:]
+    y = projection.linear(x, w)
+    assert_linear_close(y, x, w)
+    assert bits_equal(projection.linear(x, w), y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,k", [(2760, 520), (8200, 776)])
+def test_every_start_of_the_gated_walk(gpu_device, dtype, n, k):
+    """Within the two roundings of the projections and that of the gate, as for the other gated shapes."""
+    from kv_cache_repair_amd.kernels import projection
+
+    torch.manual_seed(n)
+    x = torch.randn(1, 37, k, device=gpu_device).to(dtype)
+    gate, up = ((torch.randn(n, k, device=gpu_device) * 0.05).to(dtype) for _ in range(2))
+    y = projection.silu_gate_linear(x, gate, up)
+    eager = torch.nn.functional.silu(exact_linear(x, gate)) * exact_linear(x, up)
+    assert torch.isfinite(y).all()
+    assert (ulp_distance(y, eager) <= 2).float().mean().item() >= 0.99
