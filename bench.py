@@ -834,26 +834,37 @@ def kernel_launchers(model, workload: Workload, old, old_ids, new_ids, device):
         # one "launch" = the four projections of a layer; bytes/flops averaged per kvr_linear_multi call
         out["kvr_linear_multi"] = (launch_all, total_bytes, 0, 4 * w.layers, 4)
     else:
-        # more rows than one kvr_linear_multi launch serves: the stage runs the modules' own
-        # projections (torch -> hipBLASLt): one layer's seven GEMMs at the workload's row count
+        # more rows than one kvr_linear_multi launch serves: the same four projections on the tiled kernel, each
+        # with its own split-K sum (the stage leaves the sums to their consumers)
+        from kv_cache_repair_amd.kernels import projection as proj
+
         layer = model.model.layers[0]
         a, m = layer.self_attn, layer.mlp
         x = torch.randn(b, w.hidden, device=device, generator=gen, dtype=torch.bfloat16)
         xi = torch.randn(b, w.mlp, device=device, generator=gen, dtype=torch.bfloat16)
         xo = torch.randn(b, w.hq * w.dim, device=device, generator=gen, dtype=torch.bfloat16)
-        gemms = [(mod.weight.detach(), xin) for mod, xin in ((a.q_proj, x), (a.k_proj, x), (a.v_proj, x),
-                                                             (a.o_proj, xo), (m.gate_proj, x), (m.up_proj, x),
-                                                             (m.down_proj, xi))]
-        outs = [torch.empty(b, wt.shape[0], device=device, dtype=torch.bfloat16) for wt, _ in gemms]
+        calls, nbytes, params = [], 0, 0
+        for weights, epi, xin in (
+                ([a.q_proj.weight, a.k_proj.weight, a.v_proj.weight], proj.CONCAT, x),
+                ([a.o_proj.weight], proj.CONCAT, xo),
+                ([m.gate_proj.weight, m.up_proj.weight], proj.SILU_GATE, x),
+                ([m.down_proj.weight], proj.CONCAT, xi)):
+            pl = proj.ProjectionPlan(weights, epi)
+            need = int(lib.kvr_tiled_linear_workspace_bytes(b, pl.rows, pl.k))
+            wsp = torch.empty(max(need, 1), dtype=torch.uint8, device=device)
+            y = torch.empty(b, pl.n_out, device=device, dtype=torch.bfloat16)
+            calls.append((_checked(lib.kvr_tiled_linear_multi, xin.data_ptr(), pl._count, pl._w, pl._rows, pl._ldw,
+                                   y.data_ptr(), b, pl.k, xin.stride(0), pl.n_out, epi, None, 0, wsp.data_ptr(), need,
+                                   code), (pl, xin, y, wsp)))
+            params += pl.rows * pl.k
+            nbytes += esz * (pl.rows * pl.k + b * pl.k + b * pl.n_out)
 
-        def launch_gemms():
-            for (wt, xin), y in zip(gemms, outs):
-                torch.matmul(xin, wt.t(), out=y)
-        launch_gemms.keep = (gemms, outs)
-        params = sum(wt.numel() for wt, _ in gemms)
-        nbytes = esz * (params + sum(xin.numel() + y.numel() for (_, xin), y in zip(gemms, outs)))
-        # one "launch" = the seven GEMMs of a layer; per GEMM on average
-        out["hipblaslt_projections"] = (launch_gemms, nbytes, 2 * b * params, 7 * w.layers, 7)
+        def launch_tiled():
+            for c, _ in calls:
+                c()
+        launch_tiled.keep = [c[1] for c in calls]
+        # one "launch" = the four projections of a layer; per projection on average
+        out["kvr_tiled_linear_multi"] = (launch_tiled, nbytes, 2 * b * params, 4 * w.layers, 4)
     launch_keep = (shifted, plan, qkv, q_out, cos, sin, ws, attn_out, host, dev)
     return out, launch_keep
 
@@ -923,9 +934,9 @@ def rooflines(kernels: dict, workload: str) -> tuple[dict, dict]:
     stepping = {n: k for n, k in kernels.items() if k["launches_per_step"]}
     dominant = max(stepping, key=lambda n: stepping[n]["total_us_per_step"])
     attention_bound = "mfma" if workload in ("c4", "c5") else "hbm"
-    # the bound of the dominant kernel: attention as above; hipBLASLt's projections of
-    # more than 64 rows are MFMA-bound (2*rows flops per weight element read once)
-    bound = {"kvr_packed_causal_attention": attention_bound, "hipblaslt_projections": "mfma"}.get(dominant, "hbm")
+    # the bound of the dominant kernel: attention as above; the projections of more
+    # than 64 rows (c4, c5) are MFMA-bound (2*rows flops per weight element read once)
+    bound = {"kvr_packed_causal_attention": attention_bound, "kvr_tiled_linear_multi": "mfma"}.get(dominant, "hbm")
     north = {"rotate": entry("kvr_rope_delta_rotate"), "shift_cache_build": entry("kvr_shift_cache_build"),
              "scatter": entry("kvr_indexed_scatter_kv"), "fresh_row_epilogue": entry("kvr_rope_scatter_kv"),
              "attention": entry("kvr_packed_causal_attention", attention_bound)}
