@@ -239,11 +239,15 @@ class _LayerPlans:
     desc: Any = None  # kvr_layer_desc template (no cache pointers) for kvr_decoder_layer, or None
 
 
+_TILED_MAX_ROWS = 1 << 20  # rows of one kvr_decoder_tiled_forward call
+
+
 class _PlanList(list):
     """The layers' plans of one module tree; carries the descriptor template
     that _native_layer_descs derives from them."""
 
     descs_template = None
+    tiled = None  # _tiled_weights of these plans, once asked
 
 
 _PLAN_CACHE: "weakref.WeakKeyDictionary[Any, _LayerPlans]" = weakref.WeakKeyDictionary()
@@ -788,13 +792,26 @@ def _native_layers_for(native_layers, base, plans, fused_epilogue: bool, fused_l
     return bool(native_layers)
 
 
+def _tiled_weights(plans) -> bool:
+    """Whether the tiled kernel takes every weight of the plans: k in whole 64s,
+    rows in whole 8s, rows neither overlapping nor more than 2^21 elements apart.
+    Kept with a plan list, as the weights it was built from are."""
+    ok = getattr(plans, "tiled", None)
+    if ok is None:
+        projections = [q for p in plans for q in (p.qkv, p.q, p.k, p.v, p.o, p.gate_up, p.down) if q is not None]
+        ok = all(q.k % 64 == 0 and all(rows % 8 == 0 for rows in q._rows)
+                 and all(q.k <= ld <= 1 << 21 for ld in q._ldw) for q in projections)
+        if isinstance(plans, _PlanList):
+            plans.tiled = ok
+    return ok
+
+
 def _tiled_plans_for(base, launcher: _Launcher, fused_projections, native_layers, fused_epilogue: bool,
                      fused_layers: bool, fingerprint=None):
     """Layer plans of a refresh whose layers run as one kvr_decoder_tiled_forward
     call, or None: more rows than kvr_linear_multi takes, every fusion left on
     (none asked for one by one: ``native_layers=True`` stays an error here),
-    layers with native descriptors, and the sizes that kernel tiles (a multiple
-    of 64 for every projection's k). It replaces the modules' library GEMMs at
+    layers with native descriptors, and weights that kernel takes. It replaces the modules' library GEMMs at
     every row count: 2.0x faster per call at 71 rows of a 32-layer 8B model, 1.4x
     at 282, level with them from ~1400 rows on, where the launches it saves (SiLU
     product, residual adds) make the difference."""
@@ -804,9 +821,7 @@ def _tiled_plans_for(base, launcher: _Launcher, fused_projections, native_layers
     plans = _model_plans(base, fingerprint)
     if not _native_layers_for(None, base, plans, True, True):
         return None
-    first = plans[0]
-    sizes = (first.o.n_out, launcher.q_heads * launcher.head_dim, first.down.k)
-    return None if any(size % 64 for size in sizes) else plans
+    return plans if launcher.n_sel <= _TILED_MAX_ROWS and _tiled_weights(plans) else None
 
 
 # int64 word offsets of the cache fields in kvr_layer_desc (a multiple of 8 bytes long)

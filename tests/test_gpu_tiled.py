@@ -119,6 +119,36 @@ def test_tiled_refresh_matches_the_module_path(gpu_device, family, dtype, count)
             assert cosine.min().item() >= 0.9999
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("refused", ["expanded weight", "kv rows", "row limit"])
+def test_weights_the_tiled_kernel_refuses_keep_the_module_path(gpu_device, refused, monkeypatch):
+    """What the modules served before stays served: overlapping weight rows, K/V
+    rows that are no multiple of 8, more rows than a call takes."""
+    from kv_cache_repair_amd.kernels import packed_cache as pc
+
+    model = make_model(gpu_device, "llama", kv_heads=2, head_dim=64, dtype=torch.bfloat16, layers=2)
+    if refused == "expanded weight":
+        projection = model.model.layers[1].self_attn.v_proj
+        row = projection.weight.detach()[:1].clone()
+        projection.weight = torch.nn.Parameter(row.expand(projection.weight.shape), requires_grad=False)
+    elif refused == "row limit":
+        monkeypatch.setattr(pc, "_TILED_MAX_ROWS", 95)
+    shim, ids, base = make_request(model, length=200)
+    if refused == "kv rows":
+        plans = pc._model_plans(model.model)
+        assert pc._tiled_weights(plans)
+        plans.tiled = None
+        for plan in plans:
+            plan.qkv._rows[1] = 124
+        assert not pc._tiled_weights(plans)
+        return
+    monkeypatch.setattr(pc, "_native_refresh", lambda *a, **kw: pytest.fail("native forward taken"))
+    ours, _ = pc.packed_interval_repair(shim, base, ids, [(20, 80), (100, 136)])
+    modules, _ = pc.packed_interval_repair(shim, base, ids, [(20, 80), (100, 136)], fused_projections=False)
+    for a, b in zip(ours.layers, modules.layers):
+        assert torch.equal(a.keys, b.keys) and torch.equal(a.values, b.values)
+
+
 def test_tiled_entry_points_are_exported_and_refuse_before_any_launch():
     from kv_cache_repair_amd import _native
 
