@@ -236,6 +236,7 @@ class _LayerPlans:
     down: Any
     q_cols: int
     k_cols: int
+    geometry: tuple | None = None  # _layer_geometry of the weights
     desc: Any = None  # kvr_layer_desc template (no cache pointers) for kvr_decoder_layer, or None
 
 
@@ -248,6 +249,7 @@ class _PlanList(list):
 
     descs_template = None
     tiled = None  # _tiled_weights of these plans, once asked
+    geometry = None  # _one_geometry of these plans, once asked
 
 
 _PLAN_CACHE: "weakref.WeakKeyDictionary[Any, _LayerPlans]" = weakref.WeakKeyDictionary()
@@ -317,10 +319,21 @@ def _layer_plans(layer) -> _LayerPlans | None:
         pointers=key, qkv=None if separate else plan([q, k, v]), q=plan([q]) if separate else None,
         k=plan([k]) if separate else None, v=plan([v]) if separate else None, o=plan([o]),
         gate_up=plan([gate, up], _projection.SILU_GATE), down=plan([down]), q_cols=int(q.shape[0]),
-        k_cols=int(k.shape[0]), desc=_layer_desc(layer, weights, norms))
+        k_cols=int(k.shape[0]), geometry=_layer_geometry(layer, weights), desc=_layer_desc(layer, weights, norms))
     with _PLAN_LOCK:
         _PLAN_CACHE[layer] = plans
     return plans
+
+
+def _layer_geometry(layer, weights) -> tuple | None:
+    """(query columns, K columns, head dim, hidden, intermediate) of a layer whose
+    seven weights chain as the native layer call runs them, else None."""
+    q, k, v, o, gate, up, down = (tuple(w.shape) for w in weights)
+    hidden, inter = o[0], gate[0]
+    if (q[1], k, gate, up, o[1], down) != (hidden, v, (inter, hidden), (inter, hidden), q[0], (hidden, inter)) \
+            or k[1] != hidden:
+        return None
+    return q[0], k[0], int(getattr(layer._modules["self_attn"], "head_dim", 0)), hidden, inter
 
 
 def _layer_desc(layer, weights, norms):
@@ -777,12 +790,29 @@ def _model_plans(base, fingerprint=None):
     return plans
 
 
-def _native_layers_for(native_layers, base, plans, fused_epilogue: bool, fused_layers: bool):
+def _one_geometry(plans) -> tuple | None:
+    """The _layer_geometry that all of ``plans`` share, or None. Kept with a plan
+    list, as the weights it was built from are."""
+    geometry = getattr(plans, "geometry", None)
+    if geometry is None:
+        found = {p.geometry for p in plans}
+        geometry = found.pop() if len(found) == 1 else None
+        if isinstance(plans, _PlanList):
+            plans.geometry = geometry
+    return geometry
+
+
+def _native_layers_for(native_layers, base, plans, fused_epilogue: bool, fused_layers: bool, launcher=None):
     """Whether every layer runs as one kvr_decoder_layer call. Default (None): yes
     when the projection plans, fused epilogue and fused layer ops are all in use
-    and every layer has a native descriptor and the same attention scale."""
+    and every layer has a native descriptor and the same attention scale. One
+    refresh descriptor gives the shapes of all layers, so layers of several
+    widths, or of other heads than the cache's (``launcher``), run as modules."""
     possible = (plans is not None and fused_epilogue and fused_layers
                 and all(p is not None and p.desc is not None for p in plans)
+                and _one_geometry(plans) is not None
+                and (launcher is None or _one_geometry(plans)[:3] == (
+                    launcher.q_heads * launcher.head_dim, launcher.kv_heads * launcher.head_dim, launcher.head_dim))
                 and len({float(layer._modules["self_attn"].scaling) for layer in base.layers}) == 1)
     if native_layers is None:
         return possible
@@ -819,7 +849,7 @@ def _tiled_plans_for(base, launcher: _Launcher, fused_projections, native_layers
             or launcher.n_sel <= _projection.MAX_ROWS or launcher.dtype_code == _native.DTYPE_CODES[torch.float32]):
         return None
     plans = _model_plans(base, fingerprint)
-    if not _native_layers_for(None, base, plans, True, True):
+    if not _native_layers_for(None, base, plans, True, True, launcher):
         return None
     return plans if launcher.n_sel <= _TILED_MAX_ROWS and _tiled_weights(plans) else None
 
@@ -954,7 +984,7 @@ def _refresh_into(shim, output, edited_ids_t, host_plan: IndexedPlan, layer_coun
     launcher = _launcher(device_plan, base.config, key0)
     plans = _projection_plans_for(base, fused_projections, key0.dtype, device_plan.selected_count, fingerprint)
     fused_layers = _fused_layers_for(fused_layers, key0.dtype)
-    if _native_layers_for(native_layers, base, plans, fused_epilogue, fused_layers):
+    if _native_layers_for(native_layers, base, plans, fused_epilogue, fused_layers, launcher):
         _native_refresh(base, launcher, plans, output, layer_count, edited_ids_t, positions)
         return
     tiled_plans = _tiled_plans_for(base, launcher, fused_projections, native_layers, fused_epilogue, fused_layers,

@@ -149,6 +149,28 @@ def test_weights_the_tiled_kernel_refuses_keep_the_module_path(gpu_device, refus
         assert torch.equal(a.keys, b.keys) and torch.equal(a.values, b.values)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("end", [60, 136])
+def test_layers_of_several_widths_keep_the_module_path(gpu_device, end, monkeypatch):
+    from kv_cache_repair_amd.kernels import packed_cache as pc
+
+    model = make_model(gpu_device, "llama", kv_heads=2, head_dim=64, dtype=torch.bfloat16, layers=2)
+    mlp = model.model.layers[1].mlp
+    for name, size in (("gate_proj", (384, 256)), ("up_proj", (384, 256)), ("down_proj", (256, 384))):
+        weight = torch.randn(size, device=gpu_device) * 0.03
+        getattr(mlp, name).weight = torch.nn.Parameter(weight.to(torch.bfloat16), requires_grad=False)
+    shim, ids, base = make_request(model, length=200)
+    monkeypatch.setattr(pc, "_native_refresh", lambda *a, **kw: pytest.fail("native forward taken"))
+    ours, _ = pc.packed_interval_repair(shim, base, ids, [(20, end)])
+    modules, _ = pc.packed_interval_repair(shim, base, ids, [(20, end)], fused_projections=False)
+    for a, b in zip(ours.layers, modules.layers):
+        for x, y in ((a.keys, b.keys), (a.values, b.values)):
+            if end > 84:
+                assert torch.equal(x, y)
+            # up to 64 rows each layer still runs the streaming projections: two layers' 16-bit roundings
+            assert (x.double() - y.double()).norm() <= 2 * torch.finfo(torch.bfloat16).eps * y.double().norm()
+
+
 def test_tiled_entry_points_are_exported_and_refuse_before_any_launch():
     from kv_cache_repair_amd import _native
 
