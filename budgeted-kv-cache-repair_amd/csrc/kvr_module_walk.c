@@ -23,15 +23,23 @@
  *   params         = the values of every dict's "_parameters" dict (inner then
  *                    outer, dict order; empty slots are None);
  *   dict_ids / param_ids = id() of each dict / each params entry;
- *   ptrs           = data_ptr(p) for every non-None parameter.
+ *   ptrs           = data_ptr(p) for every non-None parameter (any reader: the
+ *                    executor passes one that reads the whole layout).
  * A missing "_modules", "training", "_forward_hooks", "_forward_pre_hooks" or
  * "_parameters" entry raises KeyError, as the dict lookups they replace do.
+ *
+ * layer_constants(layers) -> tuple, six entries per decoder layer: what the
+ *   cached layer plans take from the modules besides their parameters, which the
+ *   identities above do not show when it is set anew on the same module -- the
+ *   "variance_epsilon" of input_layernorm, post_attention_layernorm, q_norm and
+ *   k_norm, the "head_dim" of self_attn, and the type of mlp's act_fn (None
+ *   where a module or entry is missing).
  */
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
 static PyObject *s_dict, *s_modules, *s_parameters, *s_training, *s_forward, *s_hf_hook, *s_fwd_hooks,
-    *s_fwd_pre_hooks;
+    *s_fwd_pre_hooks, *s_epsilon, *s_head_dim, *s_in_norm, *s_post_norm, *s_attn, *s_mlp, *s_q_norm, *s_k_norm, *s_act;
 
 static int append_dict(PyObject* out, PyObject* module) {
     PyObject* d = PyObject_GetAttr(module, s_dict);
@@ -153,10 +161,69 @@ done:
     return result;
 }
 
+/* New reference to child `name` of the module with instance dict `d` (borrowed,
+ * or NULL): the child when `name` is a submodule, else None. NULL on an error. */
+static PyObject* child(PyObject* d, PyObject* name) {
+    PyObject* mods = d && PyDict_Check(d) ? PyDict_GetItemWithError(d, s_modules) : NULL;
+    PyObject* m = mods && PyDict_Check(mods) ? PyDict_GetItemWithError(mods, name) : NULL;
+    if (!m && PyErr_Occurred()) return NULL;
+    if (!m) m = Py_None;
+    Py_INCREF(m);
+    return m;
+}
+
+/* New reference to the instance dict of child `name` of `d`, or None. */
+static PyObject* child_dict(PyObject* d, PyObject* name) {
+    PyObject* m = child(d, name);
+    if (!m || m == Py_None) return m;
+    PyObject* out = PyObject_GenericGetDict(m, NULL);
+    Py_DECREF(m);
+    return out;
+}
+
+/* Appends entry `key` of child `name` of `d` (None where either is missing). */
+static int append_entry(PyObject* out, PyObject* d, PyObject* name, PyObject* key) {
+    PyObject* cd = child_dict(d, name);
+    if (!cd) return -1;
+    PyObject* v = PyDict_Check(cd) ? PyDict_GetItemWithError(cd, key) : NULL;
+    const int rc = !v && PyErr_Occurred() ? -1 : PyList_Append(out, v ? v : Py_None);
+    Py_DECREF(cd);
+    return rc;
+}
+
+static PyObject* layer_constants(PyObject* self, PyObject* layers) {
+    PyObject* seq = PySequence_Fast(layers, "layer_constants: layers must be a sequence");
+    if (!seq) return NULL;
+    PyObject* out = PyList_New(0);
+    PyObject* result = NULL;
+    for (Py_ssize_t i = 0; out && i < PySequence_Fast_GET_SIZE(seq); ++i) {
+        PyObject* d = PyObject_GenericGetDict(PySequence_Fast_GET_ITEM(seq, i), NULL);
+        PyObject* attn = d ? child_dict(d, s_attn) : NULL;
+        PyObject* mlp = attn ? child_dict(d, s_mlp) : NULL;
+        PyObject* act = mlp ? child(mlp, s_act) : NULL;
+        const int bad = !act || append_entry(out, d, s_in_norm, s_epsilon) ||
+                        append_entry(out, d, s_post_norm, s_epsilon) || append_entry(out, attn, s_q_norm, s_epsilon) ||
+                        append_entry(out, attn, s_k_norm, s_epsilon) || append_entry(out, d, s_attn, s_head_dim) ||
+                        PyList_Append(out, act == Py_None ? Py_None : (PyObject*)Py_TYPE(act));
+        Py_XDECREF(d);
+        Py_XDECREF(attn);
+        Py_XDECREF(mlp);
+        Py_XDECREF(act);
+        if (bad) goto done;
+    }
+    if (out) result = PyList_AsTuple(out);
+done:
+    Py_XDECREF(out);
+    Py_DECREF(seq);
+    return result;
+}
+
 static PyMethodDef kMethods[] = {
     {"qualify_walk", qualify_walk, METH_VARARGS,
      "qualify_walk(model, base, data_ptr) -> (training, overridden, hooked, forward_hooked, params, dict_ids, "
      "param_ids, ptrs)"},
+    {"layer_constants", layer_constants, METH_O,
+     "layer_constants(layers) -> per layer four norm epsilons, the head dim and the activation's type"},
     {NULL, NULL, 0, NULL}};
 
 static struct PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_kvr_walk",
@@ -173,7 +240,16 @@ PyMODINIT_FUNC PyInit__kvr_walk(void) {
                  {&s_forward, "forward"},
                  {&s_hf_hook, "_hf_hook"},
                  {&s_fwd_hooks, "_forward_hooks"},
-                 {&s_fwd_pre_hooks, "_forward_pre_hooks"}};
+                 {&s_fwd_pre_hooks, "_forward_pre_hooks"},
+                 {&s_epsilon, "variance_epsilon"},
+                 {&s_head_dim, "head_dim"},
+                 {&s_in_norm, "input_layernorm"},
+                 {&s_post_norm, "post_attention_layernorm"},
+                 {&s_attn, "self_attn"},
+                 {&s_mlp, "mlp"},
+                 {&s_q_norm, "q_norm"},
+                 {&s_k_norm, "k_norm"},
+                 {&s_act, "act_fn"}};
     for (size_t i = 0; i < sizeof(names) / sizeof(names[0]); ++i)
         if (!(*names[i].slot = PyUnicode_InternFromString(names[i].text))) return NULL;
     return PyModule_Create(&kModule);

@@ -25,6 +25,10 @@
 //   the tensor's data address, as torch.Tensor.data_ptr gives it, as a builtin
 //   the executor's module walk calls for each of a model's ~290 parameters
 //   (through Python's method descriptor each call costs several times more).
+//
+// layout_key(tensor) -> bytes
+//   address, dtype, sizes and strides as int64 words: what a plan over a
+//   parameter holds of it. `p.data = view` can change all but the address.
 #include <Python.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -125,9 +129,40 @@ PyObject* data_ptr(PyObject*, PyObject* obj) {
     }
 }
 
+PyObject* layout_key(PyObject*, PyObject* obj) {
+    if (!THPVariable_Check(obj)) {
+        PyErr_SetString(PyExc_TypeError, "layout_key: expected a tensor");
+        return nullptr;
+    }
+    try {
+        const at::Tensor& t = THPVariable_Unpack(obj);
+        const auto sizes = t.sizes(), strides = t.strides();
+        const size_t n = sizes.size();
+        constexpr size_t kFew = 4;
+        int64_t few[2 + 2 * kFew];
+        std::vector<int64_t> many;
+        int64_t* words = few;
+        if (n > kFew) {
+            many.resize(2 + 2 * n);
+            words = many.data();
+        }
+        words[0] = static_cast<int64_t>(reinterpret_cast<uintptr_t>(t.const_data_ptr()));
+        words[1] = static_cast<int64_t>(t.scalar_type());
+        for (size_t i = 0; i < n; ++i) {
+            words[2 + i] = sizes[i];
+            words[2 + n + i] = strides[i];
+        }
+        return PyBytes_FromStringAndSize(reinterpret_cast<const char*>(words), static_cast<Py_ssize_t>(8 * (2 + 2 * n)));
+    } catch (const std::exception& error) {
+        PyErr_SetString(PyExc_RuntimeError, error.what());
+        return nullptr;
+    }
+}
+
 PyMethodDef kMethods[] = {
     {"kv_layers", kv_layers, METH_O, "kv_layers(layers) -> (k_ptrs, v_ptrs, first_key, uniform)"},
     {"data_ptr", data_ptr, METH_O, "data_ptr(tensor) -> int: the tensor's data address"},
+    {"layout_key", layout_key, METH_O, "layout_key(tensor) -> bytes: address, dtype, sizes and strides"},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_kvr_layout",

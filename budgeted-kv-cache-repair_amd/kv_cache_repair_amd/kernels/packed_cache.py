@@ -280,25 +280,27 @@ def _layer_modules(layer):
     return projections, norms
 
 
-def _plans_key(projections, norms) -> tuple:
+def _plans_key(layer, projections, norms) -> tuple:
     """Identity of everything a layer's plans point at: module objects, weight
-    tensors and their storage, and the projections' (absent) biases."""
-    key = []
+    tensors, their storage and layout, the projections' (absent) biases, and the
+    constants taken from the modules."""
+    layout_key = tensor_layout().layout_key
+    key = [_module_walk().layer_constants((layer,))]
     add = key.extend
     for m in (*projections, *norms):
         params = m.__dict__["_parameters"]
         w = params.get("weight")
-        add((id(m), id(w), w.data_ptr() if w is not None else 0, params.get("bias") is None))
+        add((id(m), id(w), layout_key(w) if w is not None else b"", params.get("bias") is None))
     return tuple(key)
 
 
 def _layer_plans(layer) -> _LayerPlans | None:
     """Plans for ``layer`` (one of the caller's decoder layers), cached per layer
-    and rebuilt when a module, weight or weight storage changes; None when any
+    and rebuilt when a module, weight, weight layout or constant changes; None when any
     projection has a bias, is not a plain fp16/bf16 nn.Linear, or the MLP
     activation is not SiLU."""
     projections, norms = _layer_modules(layer)
-    key = _plans_key(projections, norms)
+    key = _plans_key(layer, projections, norms)
     with _PLAN_LOCK:
         cached = _PLAN_CACHE.get(layer)
     if cached is not None and cached.pointers == key:
@@ -584,17 +586,18 @@ def _qualify(shim, edited_ids, base_cache, attention_backend, writeback_backend)
     # -1 off the GPUs, and the request device is a GPU when it matters below).
     index = device.index if device.type == "cuda" else -2
     training, overridden, hooked, forward_hooked, params, dict_ids, param_ids, ptrs = \
-        _module_walk().qualify_walk(model, base, tensor_layout().data_ptr)
+        _module_walk().qualify_walk(model, base, tensor_layout().layout_key)
     from torch.nn.modules import module as _module
 
     forward_hooked = (forward_hooked or bool(_module._global_forward_hooks)
                       or bool(_module._global_forward_pre_hooks))
     # Fingerprint of the tree: every module (its __dict__'s identity) and every
-    # parameter slot (the tensor's identity and storage address; an empty slot
-    # counts). A tree with the fingerprint that last qualified on this GPU has
-    # the same parameter tensors at the same addresses, so their device check
-    # holds as it did; the layer plans are reused under the same condition.
-    fingerprint = (dict_ids, param_ids, ptrs)
+    # parameter slot (the tensor's identity, storage address and layout; an empty
+    # slot counts), and the layers' constants by value. A tree with the
+    # fingerprint that last qualified on this GPU has the same parameter tensors
+    # at the same addresses, so their device check holds as it did; the layer
+    # plans are reused under the same condition.
+    fingerprint = (dict_ids, param_ids, ptrs, _module_walk().layer_constants(list(base.layers)))
     with _PLAN_LOCK:
         previous = _QUALIFIED.get(base)
     if previous is not None and previous[1] == index and previous[0] == fingerprint:

@@ -171,6 +171,35 @@ def test_layers_of_several_widths_keep_the_module_path(gpu_device, end, monkeypa
             assert (x.double() - y.double()).norm() <= 2 * torch.finfo(torch.bfloat16).eps * y.double().norm()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("end", [60, 136])
+@pytest.mark.parametrize("change", ["epsilon", "activation", "rows"])
+def test_refreshes_follow_what_changes_on_the_same_modules(gpu_device, change, end):
+    """Set on modules and parameters that stay the same objects at the same
+    addresses, between two refreshes: seen as the modules see it."""
+    from kv_cache_repair_amd.kernels import packed_cache as pc
+
+    model = make_model(gpu_device, "llama", kv_heads=2, head_dim=64, dtype=torch.bfloat16, layers=2)
+    shim, ids, base = make_request(model, length=200)
+    intervals = [(20, end)]
+    before, _ = pc.packed_interval_repair(shim, base, ids, intervals)
+    layer = model.model.layers[0]
+    if change == "epsilon":
+        layer.post_attention_layernorm.variance_epsilon = 0.5
+    elif change == "activation":
+        layer.mlp.act_fn = torch.nn.ReLU().eval()
+    else:
+        for mlp in (each.mlp for each in model.model.layers):
+            mlp.gate_proj.weight.data = mlp.gate_proj.weight.data[:256]
+            mlp.up_proj.weight.data = mlp.up_proj.weight.data[:256]
+            mlp.down_proj.weight.data = mlp.down_proj.weight.data[:, :256]
+    ours, _ = pc.packed_interval_repair(shim, base, ids, intervals)
+    modules, _ = pc.packed_interval_repair(shim, base, ids, intervals, fused_projections=False)
+    x, y, z = (cache.layers[1].values[0, :, 20:end].double() for cache in (ours, modules, before))
+    tight = 2 * torch.finfo(torch.bfloat16).eps * y.norm()  # two layers' 16-bit roundings
+    assert (x - y).norm() <= tight < 0.5 * (z - y).norm()
+
+
 def test_tiled_entry_points_are_exported_and_refuse_before_any_launch():
     from kv_cache_repair_amd import _native
 

@@ -58,3 +58,73 @@ def test_layers_of_several_widths_run_as_modules(base, narrow):
 def test_weights_that_do_not_chain_run_as_modules(base, change):
     resize(base.layers[1], *change)
     assert not native(base)
+
+
+def constants(layers):
+    out = []
+    for layer in layers:
+        attn, mlp = layer.self_attn, layer.mlp
+        out += [getattr(getattr(m, name, None), "variance_epsilon", None)
+                for m, name in ((layer, "input_layernorm"), (layer, "post_attention_layernorm"), (attn, "q_norm"),
+                                (attn, "k_norm"))]
+        act = getattr(mlp, "act_fn", None)
+        out += [getattr(attn, "head_dim", None), None if act is None else type(act)]
+    return tuple(out)
+
+
+@pytest.mark.parametrize("base", ["llama", "qwen3"], indirect=True)
+def test_layer_constants_match_the_attribute_reads(base):
+    walk = pc._module_walk()
+    assert walk.layer_constants(base.layers) == constants(base.layers)
+    base.layers[1].mlp.act_fn = torch.nn.GELU()
+    base.layers[2].input_layernorm.variance_epsilon = 0.25
+    base.layers[0].self_attn.head_dim = 3
+    assert walk.layer_constants(list(base.layers)) == constants(base.layers)
+    base.layers[0].mlp = torch.nn.Identity()
+    del base.layers[1].input_layernorm.variance_epsilon
+    assert walk.layer_constants(base.layers) == constants(base.layers)
+    assert walk.layer_constants([]) == ()
+    with pytest.raises(TypeError):
+        walk.layer_constants(3)
+    with pytest.raises(AttributeError):
+        walk.layer_constants([object()])
+
+
+def test_layout_key_tells_every_view_of_a_storage_apart():
+    from kv_cache_repair_amd.kernels.executor import tensor_layout
+
+    key = tensor_layout().layout_key
+    w = torch.randn(6, 6)
+    views = [w, w[:4], w[:, :4], w.t(), w[:4, :4], w.view(36), w.view(2, 3, 2, 3, 1), w.view(torch.int32), w[1:],
+             w[:, 1:], torch.randn(6, 6)]
+    assert len({key(v) for v in views}) == len(views)
+    assert key(w.view(6, 6)) == key(w) == key(torch.nn.Parameter(w, requires_grad=False))
+    with pytest.raises(TypeError, match="expected a tensor"):
+        key(None)
+
+
+@pytest.mark.parametrize("change", ["epsilon", "activation", "rows", "stride"])
+def test_plans_follow_what_changes_on_the_same_modules(base, change):
+    """The modules, parameters and addresses stay: only a constant, the activation or
+    a weight's view is set anew."""
+    layer = base.layers[1]
+    first = pc._layer_plans(layer)
+    assert pc._layer_plans(layer) is first
+    mlp = layer.mlp
+    if change == "epsilon":
+        layer.post_attention_layernorm.variance_epsilon = 0.5
+        assert pc._layer_plans(layer).desc.eps_post == 0.5
+    elif change == "activation":
+        mlp.act_fn = torch.nn.GELU()
+        assert pc._layer_plans(layer) is None
+    elif change == "rows":
+        for proj in (mlp.gate_proj, mlp.up_proj):
+            proj.weight.data = proj.weight.data[:64]
+        mlp.down_proj.weight.data = mlp.down_proj.weight.data[:, :64]
+        plans = pc._layer_plans(layer)
+        assert plans.gate_up.n_out == plans.down.k == 64 and plans.desc.ld_down == 128
+        assert not native(base)
+    else:
+        proj = layer.self_attn.q_proj
+        proj.weight.data = proj.weight.data.as_strided((64, 64), (32, 1))
+        assert pc._layer_plans(layer).desc.ld_q == 32
