@@ -268,12 +268,15 @@ def _plain_linear(module) -> bool:
 
 def _layer_modules(layer):
     """(projection modules, norm modules) of a Llama/Qwen3 decoder layer, read
-    through the `_modules` dicts (plain dict lookups: this runs per layer and
-    per refresh)."""
+    through the `_modules` dicts (plain dict lookups: this runs per layer), or
+    None when one of the projections is not there (another attention or MLP put
+    in the layer, which runs as the module it is)."""
     attention, mlp = layer._modules["self_attn"], layer._modules["mlp"]
     am, mm = attention._modules, mlp._modules
-    projections = (am["q_proj"], am["k_proj"], am["v_proj"], am["o_proj"], mm["gate_proj"], mm["up_proj"],
-                   mm["down_proj"])
+    projections = (*map(am.get, ("q_proj", "k_proj", "v_proj", "o_proj")),
+                   *map(mm.get, ("gate_proj", "up_proj", "down_proj")))
+    if None in projections:
+        return None
     norms = [layer._modules["input_layernorm"], layer._modules["post_attention_layernorm"]]
     if am.get("q_norm") is not None:
         norms += [am["q_norm"], am["k_norm"]]
@@ -297,9 +300,12 @@ def _plans_key(layer, projections, norms) -> tuple:
 def _layer_plans(layer) -> _LayerPlans | None:
     """Plans for ``layer`` (one of the caller's decoder layers), cached per layer
     and rebuilt when a module, weight, weight layout or constant changes; None when any
-    projection has a bias, is not a plain fp16/bf16 nn.Linear, or the MLP
+    projection is missing, has a bias, is not a plain fp16/bf16 nn.Linear, or the MLP
     activation is not SiLU."""
-    projections, norms = _layer_modules(layer)
+    found = _layer_modules(layer)
+    if found is None:
+        return None
+    projections, norms = found
     key = _plans_key(layer, projections, norms)
     with _PLAN_LOCK:
         cached = _PLAN_CACHE.get(layer)

@@ -128,3 +128,40 @@ def test_plans_follow_what_changes_on_the_same_modules(base, change):
         proj = layer.self_attn.q_proj
         proj.weight.data = proj.weight.data.as_strided((64, 64), (32, 1))
         assert pc._layer_plans(layer).desc.ld_q == 32
+
+
+class TwoMatrixMlp(torch.nn.Module):
+    """A decoder MLP of another form: the packed layer runs it as it is."""
+
+    def __init__(self, hidden, inner, dtype, device=None):
+        super().__init__()
+        self.fc1 = torch.nn.Linear(hidden, inner, dtype=dtype, device=device)
+        self.fc2 = torch.nn.Linear(inner, hidden, dtype=dtype, device=device)
+        self.act_fn = torch.nn.GELU()
+
+    def forward(self, x):
+        return self.fc2(self.act_fn(self.fc1(x)))
+
+
+def test_an_mlp_without_the_three_projections_has_no_plans(base):
+    base.layers[1].mlp = TwoMatrixMlp(64, 96, torch.bfloat16).eval()
+    assert [plans is None for plans in pc._model_plans(base)] == [False, True, False]
+    assert not native(base)
+    base.layers[2].mlp._modules["up_proj"] = None
+    assert pc._layer_plans(base.layers[2]) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("end", [60, 136])
+def test_refresh_runs_an_mlp_of_another_form(gpu_device, end):
+    from test_gpu_packed import make_model, make_request
+
+    model = make_model(gpu_device, "llama", kv_heads=2, head_dim=64, dtype=torch.bfloat16, layers=2)
+    model.model.layers[1].mlp = TwoMatrixMlp(256, 384, torch.bfloat16, gpu_device).eval()
+    shim, ids, base = make_request(model, length=200)
+    ours, _ = pc.packed_interval_repair(shim, base, ids, [(20, end)])
+    modules, _ = pc.packed_interval_repair(shim, base, ids, [(20, end)], fused_projections=False)
+    for a, b in zip(ours.layers, modules.layers):
+        for x, y in ((a.keys, b.keys), (a.values, b.values)):
+            # one layer of the default path up to 64 rows: the streaming projections' summation order
+            assert (x.double() - y.double()).norm() <= 2 * torch.finfo(torch.bfloat16).eps * y.double().norm()
