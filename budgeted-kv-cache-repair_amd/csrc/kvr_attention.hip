@@ -2167,29 +2167,38 @@ int64_t schedule_span(const std::vector<GroupKeys>& keys, std::vector<Chunk>& ch
 }
 
 // Modelled time (us) of a schedule of the small-row launches, for the choice of
-// the group size: per 128-key step and block of each kernel, its fixed part,
-// 0.3 us per MB of partials and a merge launch of 3 us plus 0.2 us per chunk of
-// its longest chain. Fitted to 210 measured launches (16 to 2048 rows over 2k
-// to 32k keys; 32/8 and 16/4 heads by 4, 16/8 and 8/4 by 2; head dims 64 and
-// 128): the choice costs 0.2% over the fastest group size on average. Where it
-// leaves the 16-row groups: four heads, 400 rows over 16k keys 150 -> 89 us,
-// 805 over 32k 478 -> 297 us; two heads, 282 rows over 8k keys 95 -> 38 us.
+// the group size: per 128-key step, attended row tile of a step (as the share of
+// the group's tiles) and block of each kernel, its fixed part, 0.3 us per MB of
+// partials and a merge launch of 3 us plus 0.2 us per chunk of its longest chain.
+// Fitted to measured launches of 17 to 4096 rows (spread, in runs, at the end) over
+// 512 to 32k keys, by 1 to 8 KV heads of 2, 4, 6, 8 and 10 query heads. 16-row
+// groups stay unless another size is faster by group_gain: of 4350 shapes measured
+// with every group size, five are then more than 3% slower than with 16 rows (42.5
+// -> 47.9 us the most), where one time per step and no margin made 31 slower, by up
+// to 21%. They are 5% (four heads) and 37% (two) faster on average: four heads, 400
+// rows over 16k keys 150 -> 89 us, 805 over 32k 478 -> 297 us; two heads, 282 rows
+// over 8k keys 95 -> 38 us.
 struct StepTimes {
-    double step, block, fixed;
+    double step, tiles, block, fixed;
 };
 
-StepTimes step_times(int qt, int head_dim, int group_rows) {
+StepTimes step_times(int qt, int head_dim, int group_rows, bool rounded) {
     const bool wide = head_dim == 128;
-    if (qt == 4) {
-        // between the times with rounded (1.25, 2.82 at head dim 128) and hi + lo
-        // probabilities (1.53, 3.87): the schedule does not depend on that
-        if (group_rows == kTileGroupRows) return {wide ? 1.39 : 0.92, 5.0, 0.0};
-        return {wide ? 3.25 : 2.4, 3.0, 1.0};
+    if (qt == 4) {  // rounded probabilities spare a third of the PV products
+        if (group_rows == kTileGroupRows) {
+            if (rounded) return wide ? StepTimes{1.26, 0, 5.2, 0} : StepTimes{0.88, 0, 3.0, 0};
+            return wide ? StepTimes{1.56, 0, 4.8, 0} : StepTimes{1.11, 0, 2.7, 0};
+        }
+        if (rounded) return wide ? StepTimes{1.45, 2.35, 3.4, 0} : StepTimes{1.66, 1.20, 0, 2.9};
+        return wide ? StepTimes{1.80, 2.95, 3.0, 0} : StepTimes{2.10, 1.60, 0, 1.8};
     }
-    if (group_rows == kTileGroupRows) return {wide ? 2.69 : 1.31, 3.0, 0.0};  // split-key tile kernel
-    if (group_rows == kHalfGroupRows) return {wide ? 1.55 : 1.15, 5.0, 2.0};
-    return {wide ? 2.72 : 2.23, 3.0, 2.0};
+    if (group_rows == kTileGroupRows) return {wide ? 2.69 : 1.31, 0, 3.0, 0};  // split-key tile kernel
+    if (group_rows == kHalfGroupRows) return {wide ? 1.55 : 1.15, 0, 5.0, 2.0};
+    return {wide ? 2.72 : 2.23, 0, 3.0, 2.0};
 }
+
+// The modelled share of the 16-row groups' time that another size has to stay under.
+double group_gain(int qt) { return qt == 4 ? 0.96 : 0.93; }
 
 int64_t partial_bytes(const std::vector<Chunk>& chunks, int64_t n_groups, int32_t n_q_heads, int group_rows,
                       int32_t head_dim) {
@@ -2198,14 +2207,21 @@ int64_t partial_bytes(const std::vector<Chunk>& chunks, int64_t n_groups, int32_
 }
 
 // Each block goes to the CU (of the `cus` of its head's XCD) that frees first.
-double schedule_us(const std::vector<Chunk>& chunks, int64_t n_groups, int64_t cus, const StepTimes& t,
-                   int64_t partials) {
+double schedule_us(const std::vector<GroupKeys>& keys, const std::vector<Chunk>& chunks, int64_t cus, int group_rows,
+                   const StepTimes& t, int64_t partials) {
     std::vector<double> load(static_cast<size_t>(cus), 0.0);
-    std::vector<int32_t> count(static_cast<size_t>(n_groups), 0);
+    std::vector<int32_t> count(keys.size(), 0);
     int32_t chain = 0;
+    constexpr int64_t kStep = 2 * kSub;
     for (const Chunk& c : chunks) {
+        const int64_t steps = ceil_div(c.end - c.begin, kStep);
+        int64_t attended = 0;
+        for (int i = 0; i < group_rows / kRowTile; ++i) {
+            const int64_t seen = keys[c.group].tile_kmax[i] - c.begin;
+            attended += seen > 0 ? std::min<int64_t>(ceil_div(seen, kStep), steps) : 0;
+        }
         auto least = std::min_element(load.begin(), load.end());
-        *least += ceil_div(c.end - c.begin, 2 * kSub) * t.step + t.block;
+        *least += steps * t.step + t.tiles * attended * kRowTile / group_rows + t.block;
         chain = std::max(chain, ++count[c.group]);
     }
     double us = *std::max_element(load.begin(), load.end()) + t.fixed;
@@ -2330,9 +2346,10 @@ extern "C" int64_t kvr_attention_schedule_ex(const int64_t* positions, int64_t n
     const int64_t heads = static_cast<int64_t>(n_kv_heads) * n_head_groups;
     // Few rows (64-row groups x heads fill under half the grid): smaller groups
     // need fewer key chunks each for the same grid and write less partial data;
-    // larger ones do more matrix work per K/V step (a step of 16 rows takes 0.3
-    // to 0.6 of the time of one of 64). Which wins depends on rows, keys and
-    // heads, so the schedules are compared by modelled time (schedule_us).
+    // larger ones do more matrix work per K/V step. A step of 16 rows takes 0.3 of
+    // the time of one of 64 with four heads (0.6 and 0.8 with two, at head dims 64
+    // and 128). Which wins depends on rows, keys and heads, so the schedules are
+    // compared by modelled time (schedule_us).
     const int64_t wide_units = (n_sel + kGroupRows - 1) / kGroupRows * heads;
     const bool few = mfma && 2 * wide_units <= kTargetBlocks;
     int group_rows = few ? kTileGroupRows : kGroupRows;
@@ -2483,13 +2500,13 @@ extern "C" int64_t kvr_attention_schedule_ex(const int64_t* positions, int64_t n
         }
     } else {
         chunks = balanced();
-        if (few && qt >= 2) {
+        if (few && qt >= 2 && n_sel > kTileGroupRows) {  // (up to 16 rows are one group at any size)
             const int64_t cus = kTargetBlocks / heads > 1 ? kTargetBlocks / heads : 1;
             auto rate = [&](const std::vector<Chunk>& c) {
-                return schedule_us(c, n_groups, cus, step_times(qt, head_dim, group_rows),
+                return schedule_us(keys, c, cus, group_rows, step_times(qt, head_dim, group_rows, p_rounded != 0),
                                    partial_bytes(c, n_groups, n_q_heads, group_rows, head_dim));
             };
-            double least = rate(chunks);
+            double least = rate(chunks) * group_gain(qt);
             std::vector<GroupKeys> best_keys = keys;
             int best_rows = group_rows;
             for (int rows : {kHalfGroupRows, kGroupRows}) {
