@@ -241,6 +241,7 @@ class _LayerPlans:
 
 
 _TILED_MAX_ROWS = 1 << 20  # rows of one kvr_decoder_tiled_forward call
+_TILED_WIDE, _TILED_WIDE_ROWS = 8192, 4096  # hidden size and rows from which the library's GEMMs are at least as fast
 
 
 class _PlanList(list):
@@ -850,15 +851,19 @@ def _tiled_plans_for(base, launcher: _Launcher, fused_projections, native_layers
     """Layer plans of a refresh whose layers run as one kvr_decoder_tiled_forward
     call, or None: more rows than kvr_linear_multi takes, every fusion left on
     (none asked for one by one: ``native_layers=True`` stays an error here),
-    layers with native descriptors, and weights that kernel takes. It replaces the modules' library GEMMs at
-    every row count: 2.0x faster per call at 71 rows of a 32-layer 8B model, 1.4x
-    at 282, level with them from ~1400 rows on, where the launches it saves (SiLU
-    product, residual adds) make the difference."""
+    layers with native descriptors, weights that kernel takes, and a size at which
+    it is not slower than the modules' library GEMMs. Measured per call in bf16 at
+    65 to 15104 rows of hidden sizes 1024 to 8192 (fp16 within 2% of it): 1.6 to
+    5.8x faster at 65 rows, 1.2 to 4.6x at 512, 1.0 to 2.7x at 2048, 0.98 to 1.25x
+    above for up to 5120 wide. At 8192 wide it runs from 0.95 to 1.11x from 4096
+    rows on, level on average: there the modules stay."""
     if (native_layers is not None or fused_projections not in (None, True) or not fused_epilogue or not fused_layers
             or launcher.n_sel <= _projection.MAX_ROWS or launcher.dtype_code == _native.DTYPE_CODES[torch.float32]):
         return None
     plans = _model_plans(base, fingerprint)
     if not _native_layers_for(None, base, plans, True, True, launcher):
+        return None
+    if _one_geometry(plans)[3] >= _TILED_WIDE and launcher.n_sel >= _TILED_WIDE_ROWS:
         return None
     return plans if launcher.n_sel <= _TILED_MAX_ROWS and _tiled_weights(plans) else None
 

@@ -130,6 +130,18 @@ def test_plans_follow_what_changes_on_the_same_modules(base, change):
         assert pc._layer_plans(layer).desc.ld_q == 32
 
 
+@pytest.mark.parametrize("hidden,rows,tiled", [(64, 4096, True), (64, 64, False), (64, 65, True), (8192, 4095, True),
+                                               (8192, 4096, False), (8192, 65, True), (8192, 15104, False),
+                                               (8128, 15104, True), (64, 1 << 20, True), (64, (1 << 20) + 1, False)])
+def test_rows_and_widths_that_run_tiled(monkeypatch, hidden, rows, tiled):
+    monkeypatch.setattr(pc._projection, "supported_weight", lambda weight: weight.ndim == 2)
+    base = LlamaForCausalLM(LlamaConfig(vocab_size=32, hidden_size=hidden, intermediate_size=128, num_hidden_layers=2,
+                                        num_attention_heads=4, num_key_value_heads=2, head_dim=16)).to(torch.bfloat16)
+    launcher = SimpleNamespace(q_heads=4, kv_heads=2, head_dim=16, n_sel=rows, dtype_code=2)
+    found = pc._tiled_plans_for(base.model, launcher, None, None, True, True)
+    assert (found is not None) == tiled
+
+
 class TwoMatrixMlp(torch.nn.Module):
     """A decoder MLP of another form: the packed layer runs it as it is."""
 
