@@ -134,7 +134,7 @@ __device__ inline float with_residual(const GemmArgs& a, float sum, int m, int c
 // features tile*kHalf + 8w + 0..7 as its rows 0..7 and the same features of up
 // as rows 8..15, so lane columns 4lj + i hold gate (lj < 2) or up (lj >= 2) of
 // feature 8w + 4(lj & 1) + i, and the SiLU pair meets in one wave.
-template <typename T, int MT, int CS, int NW>
+template <typename T, int MT, int CS, int NW, bool STAGGER>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))  // two blocks per CU
 skinny_gemm_kernel(GemmArgs a) {
     using G = gemm_t<T>;
@@ -208,19 +208,19 @@ skinny_gemm_kernel(GemmArgs a) {
     // 2 KB per-wave LDS tile (pieces XOR-swizzled by row: conflict-free).
     const int klast = klen - 8;
     const int chunks = (klen + kChunk - 1) / kChunk;
-    // Position c of the walk is chunk (first + c) mod chunks of the slice: blocks
-    // kPhaseRows streamed rows (gated: features) apart start kSliceChunk apart,
-    // so that they do not all read at the same offset of their weight rows at
-    // once (gate/up of an 8B model over 37 rows 42.6 -> 39.6 us = 5.9 TB/s; the
-    // 32 layers of a 64-row refresh 4.74 -> 4.52 ms). The start depends on the
-    // row's place in the launch (gated: the feature's), not on its block width,
-    // so the gated launch sums gate and up in the order of their own launches of
-    // the same split.
+    // STAGGER: position c of the walk is chunk (first + c) mod chunks, where blocks
+    // kPhaseRows streamed rows (gated: features) apart start kSliceChunk apart, so
+    // that they do not all read at the same offset of their weight rows at once.
+    // The start depends on the row's place in the launch (gated: the feature's),
+    // not on its block width, so the gated launch sums gate and up in the order of
+    // their own launches of the same split. Past the last position the chunk lies
+    // behind the slice: its loads are clamped to the slice's last 8 elements.
     const int first_row = tile * (a.gated ? kHalf : kTileN);
-    const int first = first_row / kPhaseRows % ((klen + kSliceChunk - 1) / kSliceChunk) * (kSliceChunk / kChunk);
+    const int first =
+        STAGGER ? first_row / kPhaseRows % ((klen + kSliceChunk - 1) / kSliceChunk) * (kSliceChunk / kChunk) : 0;
     auto chunk_at = [&](int c) __attribute__((always_inline)) -> int {
-        const int at = first + c;  // c <= chunks: at most one turn
-        return at >= chunks ? at - chunks : at;
+        const int at = first + c;  // at most one turn
+        return STAGGER && c >= chunks ? chunks : STAGGER && at >= chunks ? at - chunks : at;
     };
     u32x4 wf[kRing];
     const char* wrow[2] = {row_ptr(lane >> 3), row_ptr(8 + (lane >> 3))};
@@ -272,9 +272,8 @@ skinny_gemm_kernel(GemmArgs a) {
     // Chunk c: issue chunk c + 1's x loads, multiply chunk c pair by pair
     // (copy the pair's two loads into the transpose tile, refill their slots
     // with the next chunk's loads, read back the two A fragments, run the
-    // MFMAs), then store chunk c + 1 into the other buffer. After the last chunk
-    // the walk comes round to its first: those loads go into the idle buffer and
-    // unread slots.
+    // MFMAs), then store chunk c + 1 into the other buffer. Past the last chunk
+    // the loads go into the idle buffer and unread slots.
     // sched_barrier pins the loads where they are written: left alone, the
     // scheduler sinks them to the end of the chunk and exposes their latency.
     for (int c = 0; c < chunks; ++c) {
@@ -434,13 +433,28 @@ bool allow_lds(F fn, size_t bytes) {
                                static_cast<int>(bytes)) == hipSuccess;
 }
 
+template <typename T, int MT, int CS, int NW, bool STAGGER>
+int launch_walk(const GemmArgs& a, dim3 grid, hipStream_t s) {
+    constexpr size_t lds = ChunkCfg<CS, NW>::kLdsBytes;
+    static const bool ok = allow_lds(skinny_gemm_kernel<T, MT, CS, NW, STAGGER>, lds);
+    if (!ok) return KVR_E_LAUNCH_FAILED;
+    skinny_gemm_kernel<T, MT, CS, NW, STAGGER><<<grid, 64 * NW, lds, s>>>(a);
+    return KVR_OK;
+}
+
+// Blocks stagger their k offsets where all of a launch would read at the same one
+// of weight rows that are whole 4 KB long, or long: gate/up of an 8B model over 37
+// rows 42.6 -> 39.6 us (5.9 TB/s), 2048 to 28672 k 2 to 28% faster over 7168 to
+// 57344 rows. Otherwise it costs 1 to 5%: the blocks of a K split lie apart as they
+// are (5120 x 5120 over 64 rows 20.2 -> 21.3 us), rows of 2560, 3072 or 5120 k
+// do not meet (28672 gated x 2560 51.5 -> 52.9), short ones end too soon (28672
+// gated x 1024 29.3 -> 30.9).
+bool staggered(const GemmArgs& a) { return a.splits == 1 && (a.k % 2048 == 0 || a.k >= 6656); }
+
 template <typename T, int MT, int CS, int NW>
 int launch_cs(const GemmArgs& a, dim3 grid, hipStream_t s) {
-    constexpr size_t lds = ChunkCfg<CS, NW>::kLdsBytes;
-    static const bool ok = allow_lds(skinny_gemm_kernel<T, MT, CS, NW>, lds);
-    if (!ok) return KVR_E_LAUNCH_FAILED;
-    skinny_gemm_kernel<T, MT, CS, NW><<<grid, 64 * NW, lds, s>>>(a);
-    return KVR_OK;
+    return staggered(a) ? launch_walk<T, MT, CS, NW, true>(a, grid, s)
+                                             : launch_walk<T, MT, CS, NW, false>(a, grid, s);
 }
 
 template <typename T, int MT>
