@@ -236,7 +236,7 @@ class _LayerPlans:
     down: Any
     q_cols: int
     k_cols: int
-    geometry: tuple | None = None  # _layer_geometry of the weights
+    geometry: tuple | None = None  # _set_geometry
     desc: Any = None  # kvr_layer_desc template (no cache pointers) for kvr_decoder_layer, or None
 
 
@@ -328,21 +328,22 @@ def _layer_plans(layer) -> _LayerPlans | None:
         pointers=key, qkv=None if separate else plan([q, k, v]), q=plan([q]) if separate else None,
         k=plan([k]) if separate else None, v=plan([v]) if separate else None, o=plan([o]),
         gate_up=plan([gate, up], _projection.SILU_GATE), down=plan([down]), q_cols=int(q.shape[0]),
-        k_cols=int(k.shape[0]), geometry=_layer_geometry(layer, weights), desc=_layer_desc(layer, weights, norms))
+        k_cols=int(k.shape[0]), desc=_layer_desc(layer, weights, norms))
+    _set_geometry(plans, int(getattr(layer._modules["self_attn"], "head_dim", 0)))
     with _PLAN_LOCK:
         _PLAN_CACHE[layer] = plans
     return plans
 
 
-def _layer_geometry(layer, weights) -> tuple | None:
-    """(query columns, K columns, head dim, hidden, intermediate) of a layer whose
-    seven weights chain as the native layer call runs them, else None."""
-    q, k, v, o, gate, up, down = (tuple(w.shape) for w in weights)
-    hidden, inter = o[0], gate[0]
-    if (q[1], k, gate, up, o[1], down) != (hidden, v, (inter, hidden), (inter, hidden), q[0], (hidden, inter)) \
-            or k[1] != hidden:
-        return None
-    return q[0], k[0], int(getattr(layer._modules["self_attn"], "head_dim", 0)), hidden, inter
+def _set_geometry(plans: _LayerPlans, head_dim: int) -> None:
+    """plans.geometry = (query columns, K columns, head dim, hidden, intermediate)
+    when the layer's weights chain as the native layer call runs them."""
+    first = plans.q or plans.qkv
+    k_rows, v_rows = (plans.k.rows, plans.v.rows) if plans.qkv is None else (plans.qkv._rows[1], plans.qkv._rows[2])
+    o, gate_up, down = plans.o, plans.gate_up, plans.down
+    if (first.k, gate_up.k, down.rows, o.k, down.k, v_rows) == (o.rows, o.rows, o.rows, plans.q_cols, gate_up.n_out,
+                                                                k_rows):
+        plans.geometry = (plans.q_cols, k_rows, head_dim, o.rows, down.k)
 
 
 def _layer_desc(layer, weights, norms):
@@ -801,7 +802,7 @@ def _model_plans(base, fingerprint=None):
 
 
 def _one_geometry(plans) -> tuple | None:
-    """The _layer_geometry that all of ``plans`` share, or None. Kept with a plan
+    """The geometry (_set_geometry) that all of ``plans`` share, or None. Kept with a plan
     list, as the weights it was built from are."""
     geometry = getattr(plans, "geometry", None)
     if geometry is None:
