@@ -485,6 +485,9 @@ constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
 constexpr int32_t kMaxSplits = 8;
 constexpr int32_t kMinSplitSteps = 4;  // k of a split at least: four stages
 
+// The smallest tile, two blocks of which share a CU.
+constexpr bool smallest_tile(int bm, int bn) { return bm == 80 && bn == 64; }
+
 struct Choice {
     int32_t tile;
     int32_t splits;
@@ -506,7 +509,7 @@ Choice model_choice(int32_t m, int32_t rows, int32_t k, bool gated) {
     for (int t = 0; t < kTileCount; ++t) {
         const Tile& tile = kTiles[t];
         const int64_t tiles_m = ceil_div(m, tile.bm);
-        if (tile.bm == 80 && tile.bn == 64 && tiles_m > 1) continue;
+        if (smallest_tile(tile.bm, tile.bn) && tiles_m > 1) continue;
         const int64_t tiles = tiles_m * ceil_div(rows, tile.bn);
         const bool once = tiles_m == 1 && tile.bm <= kStreamRows;
         for (int32_t want = 1; want <= kMaxSplits; want *= 2) {
@@ -565,7 +568,10 @@ int launch_tile(const TiledArgs& a, hipStream_t s) {
     if constexpr (C::BM <= kStreamRows) {
         if (a.tiles_m == 1) return launch_tile<T, C, true>(a, s);
     }
-    return launch_tile<T, C, false>(a, s);
+    if constexpr (smallest_tile(C::BM, C::BN))
+        return KVR_E_INVALID_ARGUMENT;  // never chosen for more x tiles
+    else
+        return launch_tile<T, C, false>(a, s);
 }
 
 template <typename T>
