@@ -682,6 +682,16 @@ int tiled_linear(const void* x, int32_t n_weights, const void* const* w, const i
 
 using namespace kvr;
 
+extern "C" int kvr_internal_tiled_choice(int32_t m, int32_t rows, int32_t k, int32_t gated, int32_t out[4]) {
+    if (!out || !tiled_linear_ok(m, rows, k)) return KVR_E_UNSUPPORTED_SHAPE;
+    const Choice c = model_choice(m, rows, k, gated != 0);
+    out[0] = kTiles[c.tile].bm;
+    out[1] = kTiles[c.tile].bn;
+    out[2] = m <= kTiles[c.tile].bm && kTiles[c.tile].bm <= kStreamRows;
+    out[3] = c.splits;
+    return KVR_OK;
+}
+
 extern "C" int64_t kvr_tiled_linear_workspace_bytes(int32_t m, int32_t rows, int32_t k) {
     return tiled_workspace_bytes(m, rows, k);
 }

@@ -95,6 +95,12 @@ int tiled_linear(const void* x, int32_t n_weights, const void* const* w, const i
                  int64_t ldr, void* workspace, int64_t workspace_bytes, int32_t dtype, void* stream, bool reduce,
                  int32_t* splits_out);
 
+// {tile rows, tile columns, one x tile with its weights streamed, K splits} of the
+// kernel that tiled_linear launches for m rows of x by `rows` weight rows of k
+// (host-only; not a part of the public interface: it tells the tests which shapes
+// reach which kernel).
+extern "C" int kvr_internal_tiled_choice(int32_t m, int32_t rows, int32_t k, int32_t gated, int32_t out[4]);
+
 // Eight consecutive columns [col, col + 8) of `row` (col % 8 == 0) summed over
 // the splits in order, as fp32 (not yet rounded). The loads of up to
 // kPartialBatch splits are issued before the adds, so a few splits cost one

@@ -71,3 +71,25 @@ def test_every_group_size_agrees_with_the_fp64_oracle(gpu_device, case, dtype):
     picked = sorted(r for r in edges if 0 <= r < rows)
     assert_attention_close(actual[:, :, picked], oracle_attention(q[:, :, picked], k, v, [positions[r] for r in picked]))
     assert torch.equal(actual, ia.indexed_causal_attention(q, k, v, plan))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layouts", [("sparse", "token_major", "token_major"), ("token_major", "padded", "sparse")])
+@pytest.mark.parametrize("case", [CASES[3], CASES[4], CASES[6], CASES[7]])
+def test_group_sizes_on_layouts_of_the_generic_kernel(gpu_device, case, layouts):
+    """The schedule is made for a geometry, before any strides are seen: rows that
+    the matrix kernels do not read take its 32- and 64-row groups to the generic one."""
+    from kv_cache_repair_amd.kernels import indexed_attention as ia
+
+    heads, kv_heads, dim, rows, keys, _ = case
+    positions = spread(rows, keys, rows)
+    q, k, v = attention_problem(gpu_device, torch.bfloat16, heads, kv_heads, rows, keys, dim, layouts, seed=rows)
+    actual = ia.indexed_causal_attention(q, k, v, ia.IndexedPlan(positions, keys).to(gpu_device))
+    picked = sorted({0, 1, 15, 16, 31, 32, rows - 2, rows - 1} & set(range(rows)))
+    assert_attention_close(actual[:, :, picked], oracle_attention(q[:, :, picked], k, v, [positions[r] for r in picked]))
+    assert_attention_close(actual[:, :, rows // 2:rows // 2 + 8],
+                           oracle_attention(q[:, :, rows // 2:rows // 2 + 8], k, v, positions[rows // 2:rows // 2 + 8]))
+    plan = ia.IndexedPlan(positions, keys).to(gpu_device)
+    dense = ia.indexed_causal_attention(*(t.contiguous() for t in (q, k, v)), plan)
+    # the same sums in another order, rounded to bf16
+    torch.testing.assert_close(actual, dense, rtol=2 ** -6, atol=2 ** -9)

@@ -40,6 +40,21 @@ def tiled(x, weights, epilogue=CONCAT, residual=None):
     return y
 
 
+def assert_gate_close(y, x, gate, up):
+    """Every element of silu(x gate^T) * (x up^T) within what the roundings of the
+    two products (assert_linear_close's bound), of the activation and of the
+    result allow; |silu'| <= 1.1."""
+    eps, tiny = torch.finfo(y.dtype).eps, torch.finfo(y.dtype).tiny
+    size = x.double().abs()
+    g, u = (x.double() @ w.double().T for w in (gate, up))
+    g_off, u_off = (eps * p.abs() + 2.0 ** -20 * (size @ w.double().abs().T) for p, w in ((g, gate), (u, up)))
+    act = g * torch.sigmoid(g)
+    act_off = 1.1 * g_off + eps * act.abs() + tiny
+    bound = act_off * (u.abs() + u_off) + act.abs() * u_off
+    bound += eps * (act * u).abs() + eps * bound + tiny
+    assert ((y.double() - act * u).abs() <= bound).all()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rows", [(4096, 1024, 1024), (4096,), (264, 72, 40), (8,)])
@@ -79,8 +94,53 @@ def test_tiled_gate_matches_the_eager_chain(gpu_device, dtype, n, k, m):
     gate, up = ((torch.randn(n, k, device=gpu_device) * 0.05).to(dtype) for _ in range(2))
     y = tiled(x, [gate, up], SILU_GATE)
     eager = torch.nn.functional.silu(exact_linear(x, gate)) * exact_linear(x, up)
-    assert torch.isfinite(y).all()
+    assert_gate_close(y, x, gate, up)
     assert (ulp_distance(y, eager) <= 2).float().mean().item() >= 0.99
+
+
+def wide_model(device, family, dtype):
+    """Hidden size 1024, heads of 128: q/k/v and o split K up to some hundred rows."""
+    from transformers import LlamaConfig, LlamaForCausalLM, Qwen3Config, Qwen3ForCausalLM
+
+    kw = dict(vocab_size=97, hidden_size=1024, intermediate_size=2048, num_hidden_layers=3, num_attention_heads=8,
+              num_key_value_heads=4, head_dim=128, max_position_embeddings=512)
+    config, ctor = (LlamaConfig, LlamaForCausalLM) if family == "llama" else (Qwen3Config, Qwen3ForCausalLM)
+    torch.manual_seed(3)
+    model = ctor(config(**kw)).to(device=device, dtype=dtype).eval()
+    for name, p in model.named_parameters():  # per-head norms of their own
+        if "norm" in name:
+            p.data.copy_(1 + 0.2 * torch.randn(p.shape, device=device))
+    return model
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("family", ["llama", "qwen3"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("count", [65, 141, 282])
+def test_tiled_refresh_from_split_partials_matches_the_module_path(gpu_device, family, dtype, count):
+    """q/k/v, o and down leave split-K partials of `count` rows a split to the
+    fresh-row epilogue (per-head norms folded in or not) and the norms. (fp16 layers
+    with per-head norms project q, k and v apart and reduce them.)"""
+    from kv_cache_repair_amd import _native
+    from kv_cache_repair_amd.kernels import packed_cache as pc
+
+    lib = _native.lib()
+    assert all(lib.kvr_tiled_linear_workspace_bytes(count, n, k) > 0 for n, k in ((2048, 1024), (1024, 1024), (1024, 2048)))
+    model = wide_model(gpu_device, family, dtype)
+    shim, ids, base = make_request(model, length=400)
+    edited = ids.clone()
+    edited[0, 70:] = (edited[0, 70:] + 7) % 97
+    intervals = [(0, 3), (20, 10 + count), (380, 387)]
+    ours, _ = pc.packed_interval_repair(shim, base, edited, intervals)
+    modules, _ = pc.packed_interval_repair(shim, base, edited, intervals, fused_projections=False)
+    rows = torch.tensor([p for s, e in intervals for p in range(s, e)], device=gpu_device)
+    assert len(rows) == count
+    for a, b in zip(ours.layers, modules.layers):
+        for x, y in ((a.keys, b.keys), (a.values, b.values)):
+            u, v = x[0][:, rows].double(), y[0][:, rows].double()
+            # as in test_tiled_refresh_matches_the_module_path, and no row of a head apart
+            off = (u - v).norm(dim=-1) / v.norm(dim=-1)
+            assert (u - v).norm() <= 2 * torch.finfo(dtype).eps * v.norm() and off.max() <= 8 * torch.finfo(dtype).eps
 
 
 @pytest.mark.gpu
@@ -126,7 +186,17 @@ def test_weights_the_tiled_kernel_refuses_keep_the_module_path(gpu_device, refus
     rows that are no multiple of 8, more rows than a call takes."""
     from kv_cache_repair_amd.kernels import packed_cache as pc
 
-    model = make_model(gpu_device, "llama", kv_heads=2, head_dim=64, dtype=torch.bfloat16, layers=2)
+    if refused == "kv rows":  # one KV head of 12
+        from transformers import LlamaConfig, LlamaForCausalLM
+
+        torch.manual_seed(7)
+        model = LlamaForCausalLM(LlamaConfig(vocab_size=97, hidden_size=192, intermediate_size=256, num_hidden_layers=2,
+                                             num_attention_heads=16, num_key_value_heads=1, head_dim=12))
+        model = model.to(device=gpu_device, dtype=torch.bfloat16).eval()
+        assert not pc._tiled_weights(pc._model_plans(model.model))
+    else:
+        model = make_model(gpu_device, "llama", kv_heads=2, head_dim=64, dtype=torch.bfloat16, layers=2)
+        assert pc._tiled_weights(pc._model_plans(model.model))
     if refused == "expanded weight":
         projection = model.model.layers[1].self_attn.v_proj
         row = projection.weight.detach()[:1].clone()
@@ -134,14 +204,6 @@ def test_weights_the_tiled_kernel_refuses_keep_the_module_path(gpu_device, refus
     elif refused == "row limit":
         monkeypatch.setattr(pc, "_TILED_MAX_ROWS", 95)
     shim, ids, base = make_request(model, length=200)
-    if refused == "kv rows":
-        plans = pc._model_plans(model.model)
-        assert pc._tiled_weights(plans)
-        plans.tiled = None
-        for plan in plans:
-            plan.qkv._rows[1] = 124
-        assert not pc._tiled_weights(plans)
-        return
     monkeypatch.setattr(pc, "_native_refresh", lambda *a, **kw: pytest.fail("native forward taken"))
     ours, _ = pc.packed_interval_repair(shim, base, ids, [(20, 80), (100, 136)])
     modules, _ = pc.packed_interval_repair(shim, base, ids, [(20, 80), (100, 136)], fused_projections=False)
