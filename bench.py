@@ -512,6 +512,21 @@ def _north_star(a: torch.Tensor, b: torch.Tensor, rotated: bool = False) -> dict
     return stats
 
 
+def _scratch_attention(forward) -> torch.Tensor:
+    """The attention output [rows, q heads * head dim] of a native layer call, in its scratch
+    slab: after the normed rows, q/k/v, the normed q and k, and the rotated q, each at 256 bytes."""
+    d = forward.desc
+    qd, kd = d.q_heads * d.head_dim, d.kv_heads * d.head_dim
+    at, total = 0, 0
+    for i, cols in enumerate((d.hidden, qd + 2 * kd, qd, kd, qd, qd, d.hidden, d.hidden, d.intermediate)):
+        if i == 5:
+            at = total
+        total += (d.rows * cols * 2 + 255) // 256 * 256
+    if total != d.scratch_bytes:
+        raise RuntimeError("the native layer's scratch is laid out in another way")
+    return forward.scratch[at:at + d.rows * qd * 2].view(torch.bfloat16).view(d.rows, qd)
+
+
 @torch.no_grad()
 def teacher_forced_parity(model, new_ids, intervals, record, reference_output) -> dict:
     """Each decoder layer of this build fed the reference path's own layer input.
@@ -520,14 +535,16 @@ def teacher_forced_parity(model, new_ids, intervals, record, reference_output) -
     reference_refresh_stage with ``record``): its shifted cache, each layer's
     input hidden rows and attention output, the rotary tables. Layer i of this
     build runs once on ``inputs[i]`` over a copy of that shifted cache with the
-    executor's own launches (projection plans, fused RMSNorm, fresh-row
-    epilogue, the rounded-probability attention schedule: the Python-dispatched
-    shells, which enqueue the same kernels as the native layer call). Its fresh
-    K/V rows (scattered into the copy), its attention output and its output
-    hidden rows are compared with the reference layer's, so each layer's own
-    error is separated from the bf16 drift that accumulates over the depth.
-    Where the native layer call serves the model (<= 64 rows), kvr_decoder_layer
-    also runs each layer on the same input and must give the same bits.
+    executor's own launches: up to 64 rows the Python-dispatched shells
+    (projection plans, fused RMSNorm, fresh-row epilogue, the rounded-probability
+    attention schedule: the same kernels as the native layer call), more rows as
+    one kvr_decoder_tiled_forward call per layer, its attention output read from
+    the call's scratch. Its fresh K/V rows (scattered into the copy), its
+    attention output and its output hidden rows are compared with the reference
+    layer's, so each layer's own error is separated from the bf16 drift that
+    accumulates over the depth. Where the native layer call serves the model
+    (<= 64 rows), kvr_decoder_layer also runs each layer on the same input and
+    must give the same bits. ``path`` names what ran.
     """
     import dataclasses
 
@@ -549,7 +566,20 @@ def teacher_forced_parity(model, new_ids, intervals, record, reference_output) -
     plan = IndexedPlan(positions, n).to(device)
     launcher = pc._launcher(plan, base.config, key0)
     plans = pc._projection_plans_for(base, None, key0.dtype, len(positions))
-    attended = {}
+    tiled = None if plans is not None else pc._tiled_plans_for(base, launcher, None, None, True, True)
+    attended, hidden_out = {}, {}
+    tables = record["tables"]
+
+    def native_forward(of_plans, **kw):
+        first = base.layers[0]
+        forward = pc._NativeForward(launcher, int(first.mlp.down_proj.weight.shape[0]),
+                                    int(first.mlp.gate_proj.weight.shape[0]), float(first.self_attn.scaling), **kw)
+        forward.bind_tables(tables)
+        cache = cache_from_tensors([(l.keys.clone(), l.values.clone()) for l in shifted.layers])
+        descs = pc._native_layer_descs(of_plans, cache, n_layers)
+        for desc in descs:  # a single layer: its own input norm, none for the next
+            desc.input_normed, desc.next_norm = 0, None
+        return forward, cache, descs
 
     def recorder(fn, i):
         def run(x, *args, **kwargs):
@@ -557,36 +587,38 @@ def teacher_forced_parity(model, new_ids, intervals, record, reference_output) -
             return fn(x, *args, **kwargs)
         return run
 
-    shell_plans = None
-    if plans is not None:
-        shell_plans = [dataclasses.replace(p, o=recorder(p.o, i)) for i, p in enumerate(plans)]
-    view = pc._make_native_view(base, True, True, shell_plans)
-    if plans is None:  # the shells call the o_proj modules: wrap them in the shells only
+    if tiled is not None:
+        forward, output, descs = native_forward(tiled, tiled=True)
+        attention = _scratch_attention(forward)
+        for i in range(n_layers):
+            hidden_out[i] = record["inputs"][i].clone().contiguous()
+            _native.check(_native.lib().kvr_decoder_tiled_forward(
+                ctypes.byref(descs[i]), 1, ctypes.byref(forward.desc), hidden_out[i].data_ptr(), forward.stream),
+                "kvr_decoder_tiled_forward")
+            attended[i] = attention.clone()
+        del forward, descs
+    else:
+        shell_plans = None
+        if plans is not None:
+            shell_plans = [dataclasses.replace(p, o=recorder(p.o, i)) for i, p in enumerate(plans)]
+        view = pc._make_native_view(base, True, True, shell_plans)
+        if plans is None:  # the shells call the o_proj modules: wrap them in the shells only
+            for i, layer in enumerate(view.layers):
+                shell = layer._modules["self_attn"]
+                shell._modules["o_proj"] = recorder(shell._modules["o_proj"], i)
+        output = cache_from_tensors([(l.keys.clone(), l.values.clone()) for l in shifted.layers])
+        context = pc._PackedContext(plan.positions, n, "hip", plan, launcher)
+        cache = Cache(layers=[pc._PackedLayer(l.keys, l.values, context, "hip") for l in output.layers])
         for i, layer in enumerate(view.layers):
-            shell = layer._modules["self_attn"]
-            shell._modules["o_proj"] = recorder(shell._modules["o_proj"], i)
-    output = cache_from_tensors([(l.keys.clone(), l.values.clone()) for l in shifted.layers])
-    context = pc._PackedContext(plan.positions, n, "hip", plan, launcher)
-    cache = Cache(layers=[pc._PackedLayer(l.keys, l.values, context, "hip") for l in output.layers])
-    tables = record["tables"]
-    hidden_out = {}
-    for i, layer in enumerate(view.layers):
-        hidden_out[i] = layer(record["inputs"][i].clone(), position_embeddings=tables, past_key_values=cache,
-                              use_cache=True, sur_packed_context=context)
+            hidden_out[i] = layer(record["inputs"][i].clone(), position_embeddings=tables, past_key_values=cache,
+                                  use_cache=True, sur_packed_context=context)
     native = None
     if pc._native_layers_for(None, base, plans, True, True):
-        native_cache = cache_from_tensors([(l.keys.clone(), l.values.clone()) for l in shifted.layers])
-        first = base.layers[0]
-        forward = pc._NativeForward(launcher, int(first.mlp.down_proj.weight.shape[0]),
-                                    int(first.mlp.gate_proj.weight.shape[0]), float(first.self_attn.scaling))
-        forward.bind_tables(tables)
-        descs = pc._native_layer_descs(plans, native_cache, n_layers)
+        forward, native_cache, descs = native_forward(plans)
         same = True
         for i in range(n_layers):
-            desc = descs[i]
-            desc.input_normed, desc.next_norm = 0, None  # a single layer: its own input norm, none for the next
             h = record["inputs"][i].clone().contiguous()
-            status = _native.lib().kvr_decoder_layer(ctypes.byref(desc), ctypes.byref(forward.desc), h.data_ptr(),
+            status = _native.lib().kvr_decoder_layer(ctypes.byref(descs[i]), ctypes.byref(forward.desc), h.data_ptr(),
                                                      forward.stream)
             _native.check(status, "kvr_decoder_layer")
             same &= bool(torch.equal(h.view(torch.int16), hidden_out[i].contiguous().view(torch.int16)))
@@ -615,8 +647,9 @@ def teacher_forced_parity(model, new_ids, intervals, record, reference_output) -
                  "beyond_2e-2": sum(r[p]["beyond_2e-2"] for r in rows),
                  "beyond_2e-2_within_2ulp": all(r[p]["beyond_2e-2_within_2ulp"] for r in rows),
                  "elements": sum(r[p]["elements"] for r in rows)} for p in parts}
-    del output, cache, view
-    return {"layers": rows, "worst": worst, "native_layer_call_bit_identical": native,
+    del output
+    path = "kvr_decoder_tiled_forward" if tiled is not None else "kvr_decoder_layer" if native is not None else "modules"
+    return {"layers": rows, "worst": worst, "path": path, "native_layer_call_bit_identical": native,
             "min_cos_all": min(worst[p]["min_cos"] for p in parts)}
 
 
@@ -656,7 +689,7 @@ def parity_checks(model, shim, old, old_ids, new_ids, intervals, with_control=Tr
         "method": "every layer fed the reference path's own input for it; its fresh K/V rows and attention output "
                   "against the reference layer's",
         "north_star_gate": gate, "worst": forced["worst"],
-        "native_layer_call_bit_identical": forced["native_layer_call_bit_identical"],
+        "path": forced["path"], "native_layer_call_bit_identical": forced["native_layer_call_bit_identical"],
         "per_layer_max_abs": [{p: round(r[p]["max_abs"], 6) for p in ("k", "v", "attention")}
                               for r in forced["layers"]]}
     del ours, theirs, control

@@ -14,7 +14,7 @@ and every row the refresh does not select must be bit-identical to the
 reference's (rotated K within 0 ulp, copied V and prefix exact).
 
 The teacher-forced test separates each layer's own error from that drift:
-every layer of this build is fed the reference path's own input for that
+every layer of this build, as a refresh of its size runs it, is fed the reference path's own input for that
 layer (recorded from one reference run) and its fresh K/V rows and attention
 output must meet the north-star gate against the reference layer's: per-row
 cosine >= 0.9999 and max-abs <= 2e-2. An element beyond 2e-2 is accepted only
@@ -99,7 +99,9 @@ def test_teacher_forced_layers_meet_the_north_star_gate(gpu_device, name):
             f"{p} max {row[p]['max_abs']:.4f} (>2e-2: {row[p]['beyond_2e-2']}) cos {row[p]['min_cos']:.6f}"
             for p in ("k", "v", "attention")), flush=True)
     assert len(result["layers"]) == workload.layers
-    if name in ("c2", "c3"):  # <= 64 rows: the product runs kvr_decoder_layer
+    # what a refresh of the workload runs: up to 64 rows kvr_decoder_layer, else the tiled forward
+    assert result["path"] == ("kvr_decoder_layer" if name in ("c2", "c3") else "kvr_decoder_tiled_forward")
+    if name in ("c2", "c3"):
         assert result["native_layer_call_bit_identical"] is True
     for row in result["layers"]:
         for part in ("k", "v", "attention"):
