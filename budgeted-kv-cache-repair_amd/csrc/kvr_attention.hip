@@ -97,7 +97,7 @@ struct AttnArgs {
     int32_t n_head_groups;
     int32_t n_groups;
     int32_t n_work;
-    int32_t group_rows;  // rows per group: kGroupRows, or kTileGroupRows (tile kernel)
+    int32_t group_rows;  // rows per group: kGroupRows, kHalfGroupRows or kTileGroupRows
     int32_t head_dim;
     int32_t out_vec;  // output rows take 8-byte stores (unit dim stride, aligned)
     int32_t p_rounded;  // the schedule permits probabilities rounded to the input dtype (H_PROB)
@@ -747,8 +747,8 @@ __global__ void __launch_bounds__(128 * QT) attn_tile_kernel(AttnArgs a) {
 // groups) every wave takes all four sub-tiles of a step. One pair (HP = 1)
 // runs groups of 32 rows in four classes and of 64 rows in two: against the
 // split-key and wide kernels, which it replaces there but for the fewest rows,
-// 805 rows over 16k keys by 16/8 heads of 64 take 103 us instead of 217, of
-// 128 134 us instead of 499.
+// a call of 805 rows over 16k keys by 16/8 heads of 64 (fp16) takes 101 us instead
+// of 208, of 128 134 us instead of 499.
 //
 // LDS holds K and V row-major, 16-byte pieces XOR-swizzled by row (piece c of
 // key row r at c ^ (r mod D/8)), so every fragment read below is free of bank

@@ -24,14 +24,15 @@
 // next reads issued one by one between the MFMAs (in a burst before them
 // 256 x 256 ran 5% slower; spread over the whole half step the last loads came
 // too late, 3-5%: three quarters is best). 16-byte pieces are swizzled by row
-// (no bank conflicts measured).
+// (SQ_LDS_BANK_CONFLICT counts none).
 //
-// Measured (us; hipBLASLt's separate q, k, v, o, gate, up, down, SiLU and
-// residual launches of one 8B layer in brackets): 71 rows 92 (210), 141 rows
-// 112 (230), 282 rows 161 (270), 512 rows 211 (310), 1383 rows 545 (560). Rates:
-// gate/up at 71 rows 42.5 us = 5.5 TB/s of weights; 256 x 256 tiles 1.4-1.45
-// PFLOP/s at 4096 rows (2.05 GHz; 1.72 with the loads left out, so LDS traffic
-// and the issue slots of the loads are what is left).
+// Measured in the refreshes (us for the four projections of one 8B layer, from their
+// kernel traces): 71 rows 100, 141 rows (fp16) 123, 282 rows 182, 1383 rows (Qwen3
+// shape) 537, 15104 rows 5120 = 1.29 PFLOP/s; hipBLASLt's separate q, k, v, o, gate,
+// up, down, SiLU and residual launches, timed alone, took 210, 230, 270 and 560 for
+// the first four. Gate/up at 71 rows 44.6 us = 5.3 TB/s of weights, at 15104 rows
+// 1.31 PFLOP/s: the matrix cores are busy 69% of the cycles of an engine clock that
+// falls to 1.7 GHz; the rest are the turns of the stages and their LDS reads.
 #include "kvr_internal.h"
 
 #include <math.h>

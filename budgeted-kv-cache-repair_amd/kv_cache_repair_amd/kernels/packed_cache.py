@@ -854,10 +854,10 @@ def _tiled_plans_for(base, launcher: _Launcher, fused_projections, native_layers
     (none asked for one by one: ``native_layers=True`` stays an error here),
     layers with native descriptors, weights that kernel takes, and a size at which
     it is not slower than the modules' library GEMMs. Measured per call in bf16 at
-    65 to 15104 rows of hidden sizes 1024 to 8192 (fp16 within 2% of it): 1.6 to
-    5.8x faster at 65 rows, 1.2 to 4.6x at 512, 1.0 to 2.7x at 2048, 0.98 to 1.25x
-    above for up to 5120 wide. At 8192 wide it runs from 0.95 to 1.11x from 4096
-    rows on, level on average: there the modules stay."""
+    65 to 15104 rows of hidden sizes 1024 to 8192 (fp16 within 2% of it): 1.5 to
+    5.8x faster at 65 rows, 1.1 to 4.6x at 512, 0.97 to 2.7x at 2048, 0.95 to 1.25x
+    above for up to 5120 wide (1.07x on average). At 8192 wide it runs at 0.95 to
+    1.11x from 4096 rows on, level on average: there the modules stay."""
     if (native_layers is not None or fused_projections not in (None, True) or not fused_epilogue or not fused_layers
             or launcher.n_sel <= _projection.MAX_ROWS or launcher.dtype_code == _native.DTYPE_CODES[torch.float32]):
         return None

@@ -13,8 +13,12 @@ extern "C" {
 
 /*
  * The projections of kvr_linear_multi for more rows (any m up to 2^20), by a
- * kernel that tiles x and the weights through LDS: same operands, epilogues,
- * rounding and determinism. k is a multiple of 64 and every weight's row count
+ * kernel that tiles x and the weights through LDS: same operands, epilogues and
+ * rounding, the same bits from call to call. The order of a sum over k depends on m
+ * and on all the weights of the call (tile, K split and the start of the walk over
+ * k follow from them): other calls over the same row, kvr_linear_multi's, and for
+ * the gated epilogue two separate projections with kvr_silu_mul, agree up to the
+ * order of their fp32 sums. k is a multiple of 64 and every weight's row count
  * a multiple of 8; ldx and ldw are multiples of 8 elements (at most 2^21) on
  * 16-byte aligned bases, ldy and ldr multiples of 4 on 8-byte aligned ones;
  * `workspace` (16-byte aligned) has kvr_tiled_linear_workspace_bytes(m, rows
