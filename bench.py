@@ -924,7 +924,8 @@ def measure_kernels(model, workload, old, old_ids, new_ids, device) -> dict:
 TRAFFIC_SUMMARIES = tuple(sorted((ROOT / "profiles").glob("*.md")))
 KERNEL_SOURCES = {"kvr_packed_causal_attention": "kvr_attention.hip", "kvr_shift_cache_build": "kvr_rotate.hip",
                   "kvr_rope_delta_rotate": "kvr_rotate.hip", "kvr_indexed_scatter_kv": "kvr_scatter.hip",
-                  "kvr_rope_scatter_kv": "kvr_fresh.hip", "kvr_linear_multi": "kvr_gemm.hip"}
+                  "kvr_rope_scatter_kv": "kvr_fresh.hip", "kvr_linear_multi": "kvr_gemm.hip",
+                  "kvr_tiled_linear_multi": "kvr_gemm_tiled.hip"}
 
 
 def source_digest(name: str) -> str:
